@@ -1827,38 +1827,16 @@ void s2p(hipStream_t s, int kt, int nchunk, const int* tbeg, const int* tnum, co
 }
 
 // ---------------------------------------------------------------------------
-// batched indexed FP64 GEMM: 64 x 64 tile of C per block, K in steps of 16.
+// batched indexed FP64 GEMM
 //
 // These products feed or apply the truncated pseudoinverses, whose singular
 // values run down to 0.1^(np+1) of the largest: y = P x cancels massively, so
 // the rounding of a plain FP64 dot product depends on the summation order at
-// the 1e-11 (np 6) to 1e-9 (np 8) level of the final potential.  Each output
-// is therefore accumulated with the error-free transformations TwoProd (FMA)
-// and TwoSum (Knuth), i.e. the compensated dot product "Dot2" of Ogita, Rump
-// and Oishi (SIAM J. Sci. Comput. 26, 2005), and rounded once at the end.
-__device__ inline void dot2_acc(double& hi, double& lo, double a, double b)
-{
-#pragma clang fp contract(off)
-  double p = a * b;
-  double e = fma(a, b, -p);
-  double s = hi + p;
-  double bb = s - hi;
-  double t = (hi - (s - bb)) + (p - bb);
-  hi = s;
-  lo += t + e;
-}
+// the 1e-11 (np 6) to 1e-9 (np 8) level of the final potential.  The plain
+// form therefore accumulates every pseudoinverse apply in about twice FP64's
+// precision (k_gemm_cmp) and rounds once at the end.
 
-// (o + hi + lo) rounded once (up to the last TwoSum)
-__device__ inline double dot2_finish(double o, double hi, double lo)
-{
-#pragma clang fp contract(off)
-  double s = o + hi;
-  double bb = s - o;
-  double t = (o - (s - bb)) + (hi - bb);
-  return s + (t + lo);
-}
-
-template <bool DOT2>
+// 64 x 64 tile of C per block, K in steps of 16, on the VALU.
 __global__ __launch_bounds__(256) void k_gemm(GemmArgs p)
 {
   const int grp = blockIdx.z;
@@ -1871,11 +1849,11 @@ __global__ __launch_bounds__(256) void k_gemm(GemmArgs p)
   __shared__ double As[16][65];
   __shared__ double Bs[16][65];
   const int t = threadIdx.x, tx = t & 15, ty = t >> 4;
-  double hi[4][4], lo[4][4];
+  double acc[4][4];
 #pragma unroll
   for (int i = 0; i < 4; i++)
 #pragma unroll
-    for (int j = 0; j < 4; j++) hi[i][j] = lo[i][j] = 0.0;
+    for (int j = 0; j < 4; j++) acc[i][j] = 0.0;
   for (int k0 = 0; k0 < K; k0 += 16) {
 #pragma unroll
     for (int i = 0; i < 4; i++) {
@@ -1911,12 +1889,7 @@ __global__ __launch_bounds__(256) void k_gemm(GemmArgs p)
 #pragma unroll
       for (int i = 0; i < 4; i++)
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-          if (DOT2)
-            dot2_acc(hi[i][j], lo[i][j], a[i], b[j]);
-          else
-            hi[i][j] = fma(a[i], b[j], hi[i][j]);
-        }
+        for (int j = 0; j < 4; j++) acc[i][j] = fma(a[i], b[j], acc[i][j]);
     }
     __syncthreads();
   }
@@ -1930,131 +1903,275 @@ __global__ __launch_bounds__(256) void k_gemm(GemmArgs p)
     for (int i = 0; i < 4; i++) {
       int row = rb + tx + 16 * i;
       if (row >= p.M) continue;
-      double h = hi[i][j], l = lo[i][j];
-      if (p.cscale) {  // power of two: exact
-        h *= p.cscale[row];
-        l *= p.cscale[row];
-      }
-      if (DOT2)
-        out[row] = dot2_finish(p.accumulate ? out[row] : 0.0, h, l);
-      else
-        out[row] = p.accumulate ? out[row] + h : h;
+      double h = acc[i][j];
+      if (p.cscale) h *= p.cscale[row];  // power of two: exact
+      out[row] = p.accumulate ? out[row] + h : h;
     }
   }
 }
 
-// Compensated (Dot2) product, staged like k_gemm_mx: 64 x 64 tile of C per
-// block, each thread a 4 x 4 block of (hi, lo) accumulators; K in steps of 8
-// (segments are multiples of 8), the A and B tiles double-buffered in LDS with
-// the next step's values loaded into registers while the current step is
-// accumulated; each thread's staging addresses are fixed per segment (no
-// per-element index arithmetic).  One barrier per step.
-__global__ __launch_bounds__(256) void k_gemm_dot2(GemmArgs p)
+// Compensated product y = A x for the pseudoinverse applies, in about twice
+// FP64's precision at four vector operations per multiply-add.
+//
+// A running sum kept in one binade splits off its own rounding errors: with
+// hi in [2^m, 2^(m+1)) every h = fma(a, b, hi) is a multiple of the fixed
+// u = 2^(m-52), so hi - h is exact, and fma(a, b, hi - h) is the part of a b
+// that h did not take, at most u / 2, rounded to 2^-53 of itself.  lo collects
+// these.  The sum starts at sigma = 1.5 2^m and stays in the binade because
+// the columns of B are scaled by a power of two to at most 1 in magnitude (2
+// at the very top of the FP64 range) and 2^(m-2) bounds the row's sum of |A|
+// (cmp_sigma, once per operator at set-up); hi - sigma is exact and
+// (hi - sigma) + lo rounds once.  The error before that rounding is of the
+// order of K^2 2^-106 sigma, as that of a TwoProd / TwoSum dot product, which
+// takes ten operations instead of four.
+//
+// Bound by the FP64 vector rate (the matrix cores do not give out the
+// rounding errors of their sums).  A block of WM x WN x WK waves forms a
+// 32 WM x 32 WN tile, each wave 32 x 32 of it as 4 x 4 per lane (4 LDS reads
+// of 16 bytes feed 64 vector operations), the K steps of 8 double-buffered in
+// LDS; WK > 1 splits K over the block's waves, whose (hi - sigma) --
+// multiples of u, summed exactly -- and lo are added through LDS in wave
+// order, so the result does not depend on scheduling and needs no workspace
+// or second launch.
+// Measured against a TwoProd / TwoSum product on 64 x 64 tiles with no split:
+// 152 x 296 over 524,288 columns (Laplace np 6, 4M points, 16 right-hand
+// sides) 9.36 -> 3.79 ms + 0.26 ms for the scales (27 of 39 T vector
+// operations/s); 608 x 888 (Stokes np 6) over 4,100 columns 970 -> 392 us,
+// over 20 columns 437 -> 55 us; 56 x 152 (np 4) over 64 columns 80 -> 17 us.
+__device__ inline void cmp_acc(double& hi, double& lo, double a, double b)
 {
-  const int grp = blockIdx.z;
-  const int n0 = p.gbeg[grp], n1 = p.gbeg[grp + 1];
-  const long cb = (long)n0 * p.Rc + (long)blockIdx.x * 64, ce = (long)n1 * p.Rc;
-  if (cb >= ce) return;  // block-uniform
-  const int rb = blockIdx.y * 64;
-  const double* A = p.A + grp * p.a_gstride;
-  const int nstep = p.nseg * p.Kseg / 8, sps = p.Kseg / 8;
-  __shared__ double As[2][8][64];
-  __shared__ double Bs[2][8][65];
-  const int t = threadIdx.x, tx = t & 15, ty = t >> 4;
-  // staging: A elements (kk = e >> 6, row = e & 63), B elements (kk = e & 7,
-  // column e >> 3) for e = t and t + 256
-  int akk[2], arow[2], bkk[2], bcl[2], bn_n[2], bn_r[2];
-  bool aok[2], bok[2];
-#pragma unroll
-  for (int i = 0; i < 2; i++) {
-    const int e = t + 256 * i;
-    akk[i] = e >> 6;
-    arow[i] = e & 63;
-    aok[i] = rb + arow[i] < p.M;
-    bkk[i] = e & 7;
-    bcl[i] = e >> 3;
-    const long j = cb + bcl[i];
-    bok[i] = j < ce;
-    bn_n[i] = bok[i] ? (int)(j / p.Rc) : 0;
-    bn_r[i] = bok[i] ? (int)(j - (long)bn_n[i] * p.Rc) : 0;
+#pragma clang fp contract(off)
+  const double h = fma(a, b, hi);
+  lo += fma(a, b, hi - h);
+  hi = h;
+}
+
+double cmp_sigma(double abs_row_sum)
+{
+  int m = 0;
+  std::frexp(abs_row_sum, &m);  // abs_row_sum <= 2^m
+  return abs_row_sum > 0.0 ? std::ldexp(1.5, m + 2) : 1.0;
+}
+
+// e with 2^e >= m, for the largest magnitude m of a column (0 for a column
+// that is all zero or not finite, whose products are then what they are)
+__device__ inline int cmp_exp(double m)
+{
+  int e = 0;
+  if (m > 0.0 && m <= DBL_MAX) (void)frexp(m, &e);
+  return min(max(e, -1000), 1023);
+}
+
+// cmp_exp of every column of B, one wave per column
+__global__ __launch_bounds__(256) void k_gemm_cmp_exp(GemmArgs p, int* __restrict__ out)
+{
+  const long j = (long)blockIdx.x * 4 + (threadIdx.x >> 6), l = threadIdx.x & 63;
+  if (j >= (long)p.ncol * p.Rc) return;  // wave-uniform
+  const long n = j / p.Rc;
+  const double* b = p.B + ((long)p.bnode[n] * p.Rc + (j - n * p.Rc)) * p.Kseg;
+  double m = 0.0;
+  for (long k = 2 * l; k < p.Kseg; k += 128) {
+    const double2 v = *(const double2*)(b + k);
+    m = fmax(m, fmax(fabs(v.x), fabs(v.y)));
   }
-  const double* bcol[2];
-  double bmul[2];
-  auto seg_ptrs = [&](int seg) {
 #pragma unroll
-    for (int i = 0; i < 2; i++) {
-      const int bn = bok[i] ? p.bnode[(long)seg * p.ncol + bn_n[i]] : -1;
-      bcol[i] = p.B + (bn >= 0 ? ((long)bn * p.Rc + bn_r[i]) * p.Kseg : 0) + bkk[i];
-      bmul[i] = bn >= 0 ? 1.0 : 0.0;
-    }
+  for (int d = 1; d < 64; d *= 2) m = fmax(m, __shfl_xor(m, d));
+  if (l == 0) out[j] = cmp_exp(m);
+}
+
+// exps: cmp_exp of every column, or null (the block finds those of its own)
+template <int WM, int WN, int WK>
+__global__ __launch_bounds__(64 * WM * WN * WK, WK == 16 ? 4 : 3) void k_gemm_cmp(GemmArgs p,
+                                                                              const int* __restrict__ exps)
+{
+  static_assert(WK == 1 || (WM == 1 && WN == 1), "K is split between waves of one tile");
+  constexpr int NT = 64 * WM * WN * WK, NG = 64 * WM * WN;   // threads of the block, of one K part
+  constexpr int BM = 32 * WM, BN = 32 * WN, LB = BN + 8;     // LB: padded row, conflict-free staging writes
+  constexpr int NA = (BM * 4 + NG - 1) / NG, NB = BN * 4 / NG;  // 16-byte operand pairs per thread and step
+  constexpr int PART = 16 * (BM + LB);                       // LDS doubles of one K part
+  static_assert(WK == 1 || PART >= 32 * 32, "the split sums reuse the staging memory");
+  __shared__ __align__(16) double lds[WK * PART];
+  __shared__ int s_exp[BN];
+  const long cb = (long)blockIdx.x * BN, ce = (long)p.ncol * p.Rc;
+  const int rb = blockIdx.y * BM, K = p.Kseg, nstep = K / 8;
+  const int t = threadIdx.x, kg = t / NG, tg = t - kg * NG, w = tg >> 6, l = t & 63;
+  // column c of the block in B (past the end: the last one, whose copies are
+  // not stored, as are those of row 0 past the end of A)
+  auto column = [&](int c) {
+    const long j = min(cb + c, ce - 1), n = j / p.Rc;
+    return p.B + ((long)p.bnode[n] * p.Rc + (j - n * p.Rc)) * K;
   };
-  double ra[2], rbv[2];
-  auto load = [&](int st) {
-    const int k0 = st * 8, kin = (st - (st / sps) * sps) * 8;
-#pragma unroll
-    for (int i = 0; i < 2; i++) {
-      ra[i] = aok[i] ? A[(long)(k0 + akk[i]) * p.M + rb + arow[i]] : 0.0;
-      double v = bcol[i][kin] * bmul[i];
-      if (p.bscale) v *= p.bscale[kin + bkk[i]];  // power of two: exact
-      rbv[i] = v;
+  if (exps) {
+    if (t < BN) s_exp[t] = exps[min(cb + t, ce - 1)];
+  } else {
+    constexpr int TPC = NT / BN;  // adjacent threads per column
+    const double* b = column(t / TPC);
+    double m = 0.0;
+#pragma unroll 4
+    for (int k = 2 * (t % TPC); k < K; k += 2 * TPC) {
+      const double2 v = *(const double2*)(b + k);
+      m = fmax(m, fmax(fabs(v.x), fabs(v.y)));
     }
+#pragma unroll
+    for (int d = 1; d < TPC; d *= 2) m = fmax(m, __shfl_xor(m, d));
+    if (t % TPC == 0) s_exp[t / TPC] = cmp_exp(m);
+  }
+  __syncthreads();
+  const int st0 = nstep * kg / WK, st1 = nstep * (kg + 1) / WK;  // this part's K steps
+  double* const sA = lds + kg * PART;
+  double* const sB = sA + 16 * BM;
+  int ao[NA];
+  const double* bp[NB];
+  double bs[NB];
+#pragma unroll
+  for (int i = 0; i < NA; i++) {  // two rows of one K index
+    const int e = tg + NG * i, row = 2 * (e % (BM / 2)), kk = (e / (BM / 2)) & 7;
+    ao[i] = kk * p.M + (rb + row < p.M ? rb + row : 0);
+  }
+#pragma unroll
+  for (int i = 0; i < NB; i++) {  // two K indices of one column
+    const int e = tg + NG * i, c = e >> 2;
+    bp[i] = column(c) + 2 * (e & 3);
+    bs[i] = ldexp(1.0, -s_exp[c]);
+  }
+  double2 ra[NA], rbv[NB];
+  auto load = [&](int st) {
+    const double* a = p.A + (long)st * 8 * p.M;
+#pragma unroll
+    for (int i = 0; i < NA; i++) ra[i] = *(const double2*)(a + ao[i]);
+#pragma unroll
+    for (int i = 0; i < NB; i++) rbv[i] = *(const double2*)(bp[i] + st * 8);
   };
   auto store = [&](int buf) {
 #pragma unroll
-    for (int i = 0; i < 2; i++) {
-      As[buf][akk[i]][arow[i]] = ra[i];
-      Bs[buf][bkk[i]][bcl[i]] = rbv[i];
+    for (int i = 0; i < NA; i++) {
+      const int e = tg + NG * i, row = 2 * (e % (BM / 2)), kk = e / (BM / 2);
+      if (BM * 4 % NG == 0 || kk < 8) *(double2*)(sA + (buf * 8 + kk) * BM + row) = ra[i];
+    }
+#pragma unroll
+    for (int i = 0; i < NB; i++) {
+      const int e = tg + NG * i, c = e >> 2, kk = 2 * (e & 3);
+      sB[(buf * 8 + kk) * LB + c] = rbv[i].x * bs[i];
+      sB[(buf * 8 + kk + 1) * LB + c] = rbv[i].y * bs[i];
     }
   };
+  // the wave's tile of the block, and the lane's 4 x 4 of it
+  const int wr = 32 * (w % WM), wc = 32 * (w / WM), r0 = wr + 4 * (l & 7), c0 = wc + 4 * (l >> 3);
+  const bool wact = rb + wr < p.M && cb + wc < ce;  // wave-uniform
+  // M is a multiple of 8: a lane's 4 rows are all in or all past the end
+  const double* sig = p.sigma + (rb + r0 < p.M ? rb + r0 : 0);
   double hi[4][4], lo[4][4];
 #pragma unroll
   for (int i = 0; i < 4; i++)
 #pragma unroll
-    for (int j = 0; j < 4; j++) hi[i][j] = lo[i][j] = 0.0;
-  seg_ptrs(0);
-  load(0);
-  store(0);
-  __syncthreads();
-  for (int st = 0; st < nstep; st++) {
-    const int buf = st & 1;
-    const bool more = st + 1 < nstep;
-    if (more) {
-      if ((st + 1) % sps == 0) seg_ptrs((st + 1) / sps);
-      load(st + 1);
+    for (int j = 0; j < 4; j++) {
+      hi[i][j] = sig[i];
+      lo[i][j] = 0.0;
     }
-#pragma unroll 2
-    for (int kk = 0; kk < 8; kk++) {
-      double a[4], b[4];
+  if (st0 < st1) {
+    load(st0);
+    store(0);
+  }
+  __syncthreads();
+  const int nit = (nstep + WK - 1) / WK;
+  for (int it = 0; it < nit; it++) {
+    const int buf = it & 1;
+    const bool more = st0 + it + 1 < st1;
+    if (more) load(st0 + it + 1);
+    if (wact && st0 + it < st1) {
+      const double* pa = sA + buf * 8 * BM + r0;
+      const double* pb = sB + buf * 8 * LB + c0;
+#pragma unroll WK == 16 ? 2 : 8
+      for (int kk = 0; kk < 8; kk++) {
+        const double2 a0 = *(const double2*)(pa + kk * BM), a1 = *(const double2*)(pa + kk * BM + 2);
+        const double2 b0 = *(const double2*)(pb + kk * LB), b1 = *(const double2*)(pb + kk * LB + 2);
+        const double a[4] = {a0.x, a0.y, a1.x, a1.y}, b[4] = {b0.x, b0.y, b1.x, b1.y};
 #pragma unroll
-      for (int i = 0; i < 4; i++) a[i] = As[buf][kk][tx + 16 * i];
+        for (int i = 0; i < 4; i++)
 #pragma unroll
-      for (int j = 0; j < 4; j++) b[j] = Bs[buf][kk][ty + 16 * j];
-#pragma unroll
-      for (int i = 0; i < 4; i++)
-#pragma unroll
-        for (int j = 0; j < 4; j++) dot2_acc(hi[i][j], lo[i][j], a[i], b[j]);
+          for (int j = 0; j < 4; j++) cmp_acc(hi[i][j], lo[i][j], a[i], b[j]);
+      }
     }
     if (more) store(buf ^ 1);
     __syncthreads();
   }
+  auto result = [&](int c, int row, double h, double lw) {  // the scales are powers of two
+    const double v = ldexp(h + lw, s_exp[c]);
+    return p.cscale ? v * p.cscale[row] : v;
+  };
+  auto out_col = [&](int c) {
+    const long j = cb + c, n = j / p.Rc;
+    return p.C + ((long)p.cnode[n] * p.Rc + (j - n * p.Rc)) * p.M;
+  };
+  if constexpr (WK == 1) {
+    if (!wact || rb + r0 >= p.M) return;
 #pragma unroll
-  for (int j = 0; j < 4; j++) {
-    const long jj = cb + ty + 16 * j;
-    if (jj >= ce) continue;
-    const int n = (int)(jj / p.Rc), r = (int)(jj - (long)n * p.Rc);
-    double* out = p.C + ((long)p.cnode[n] * p.Rc + r) * p.M;
+    for (int j = 0; j < 4; j++) {
+      if (cb + c0 + j >= ce) continue;
+      double* out = out_col(c0 + j) + rb + r0;
+      double v[4];
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const int row = rb + tx + 16 * i;
-      if (row >= p.M) continue;
-      double h = hi[i][j], l = lo[i][j];
-      if (p.cscale) {  // power of two: exact
-        h *= p.cscale[row];
-        l *= p.cscale[row];
+      for (int i = 0; i < 4; i++) v[i] = result(c0 + j, rb + r0 + i, hi[i][j] - sig[i], lo[i][j]);
+      *(double2*)out = make_double2(v[0], v[1]);
+      *(double2*)(out + 2) = make_double2(v[2], v[3]);
+    }
+  } else {
+    constexpr int NE = (32 * 32 + NT - 1) / NT;
+    double h[NE];
+    auto spread = [&](auto&& f) {
+      double* d = lds + kg * 1024;
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        *(double2*)(d + (c0 + j) * 32 + r0) = make_double2(f(0, j), f(1, j));
+        *(double2*)(d + (c0 + j) * 32 + r0 + 2) = make_double2(f(2, j), f(3, j));
       }
-      out[row] = dot2_finish(p.accumulate ? out[row] : 0.0, h, l);
+    };
+    spread([&](int i, int j) { return hi[i][j] - sig[i]; });
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < NE; k++) {
+      h[k] = 0.0;
+#pragma unroll
+      for (int g = 0; g < WK; g++) h[k] += lds[g * 1024 + t + NT * k];
+    }
+    __syncthreads();
+    spread([&](int i, int j) { return lo[i][j]; });
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < NE; k++) {
+      const int at = t + NT * k, row = rb + (at & 31), c = at >> 5;
+      double lw = 0.0;
+#pragma unroll
+      for (int g = 0; g < WK; g++) lw += lds[g * 1024 + at];
+      if (row < p.M && cb + c < ce) out_col(c)[row] = result(c, row, h[k], lw);
     }
   }
+}
+
+// The rule by the number of 32 x 32 tiles: 768 blocks of 4 waves at 3 waves
+// per SIMD fill the chip, so below about that count K is split over 16 (8)
+// waves of one block to have enough waves at all; from there on 4 waves per
+// tile keep the blocks small and even (4,100 columns of 608 x 888: 437 us
+// against the 970 of whole 64 x 64 tiles), until 8,192 tiles, where a 32 x 128
+// tile reads each operand of B less often (4M points: 3.79 ms, 64 x 64 tiles
+// whose third row block is half empty 4.07 ms).  The scales: in the block
+// itself where there are few tiles (a launch costs as much), in a pass of
+// their own, kept in the split-K workspace, where 5 to 28 row tiles would
+// each read the columns again (608 x 888: 437 -> 376 + 7 us).
+static void gemm_cmp(hipStream_t s, const GemmArgs& a, long cols)
+{
+  const long n32 = (long)((a.M + 31) / 32) * ((cols + 31) / 32);
+  int* exps = n32 >= 640 && a.work && a.work_n * 2 >= cols ? (int*)a.work : nullptr;
+  if (exps) hipLaunchKernelGGL(k_gemm_cmp_exp, dim3((unsigned)((cols + 3) / 4)), dim3(256), 0, s, a, exps);
+  const unsigned rows = (unsigned)((a.M + 31) / 32);
+  if (n32 >= 8192)
+    hipLaunchKernelGGL((k_gemm_cmp<1, 4, 1>), dim3((unsigned)((cols + 127) / 128), rows), dim3(256), 0, s, a, exps);
+  else if (n32 >= 640)
+    hipLaunchKernelGGL((k_gemm_cmp<1, 1, 4>), dim3((unsigned)((cols + 31) / 32), rows), dim3(256), 0, s, a, exps);
+  else if (n32 >= 256)
+    hipLaunchKernelGGL((k_gemm_cmp<1, 1, 8>), dim3((unsigned)((cols + 31) / 32), rows), dim3(512), 0, s, a, exps);
+  else
+    hipLaunchKernelGGL((k_gemm_cmp<1, 1, 16>), dim3((unsigned)((cols + 31) / 32), rows), dim3(1024), 0, s, a, exps);
 }
 
 // Plain (uncompensated) form on the FP64 matrix cores: the same 64 x 64 tile
@@ -2330,10 +2447,14 @@ void gemm(hipStream_t s, const GemmArgs& a)
 {
   if (a.ngroup <= 0 || a.maxcols <= 0) return;
   long cols = (long)a.maxcols * a.Rc;
+  if (a.compensated) {
+    gemm_cmp(s, a, cols);
+    return;
+  }
   // wide tiles, with K split over blocks (partials in a.work) when the
   // columns alone give fewer than 2 blocks per CU; 64 x 64 tiles without a
   // workspace
-  if (!a.compensated && a.mfma == 2 && a.Kseg % 8 == 0) {
+  if (a.mfma == 2 && a.Kseg % 8 == 0) {
     int ks = gemm_split(a);
     if (a.B2 && !(a.work && (long)ks * a.ctot * a.M <= a.work_n)) ks = 1;  // two B buffers: wide tiles only
     if (ks == 1 || (a.work && (long)ks * a.ctot * a.M <= a.work_n)) {
@@ -2363,14 +2484,10 @@ void gemm(hipStream_t s, const GemmArgs& a)
     }
   }
   dim3 grid((unsigned)((cols + 63) / 64), (a.M + 63) / 64, a.ngroup);
-  if (a.compensated && a.Kseg % 8 == 0)
-    hipLaunchKernelGGL(k_gemm_dot2, grid, dim3(256), 0, s, a);
-  else if (a.compensated)
-    hipLaunchKernelGGL(k_gemm<true>, grid, dim3(256), 0, s, a);
-  else if (a.mfma)
+  if (a.mfma)
     hipLaunchKernelGGL(k_gemm_mfma, grid, dim3(256), 0, s, a);
   else
-    hipLaunchKernelGGL(k_gemm<false>, grid, dim3(256), 0, s, a);
+    hipLaunchKernelGGL(k_gemm, grid, dim3(256), 0, s, a);
 }
 
 // ---------------------------------------------------------------------------

@@ -121,7 +121,9 @@ struct GemmArgs {
   const double* bscale;
   const double* cscale;
   int accumulate;
-  int compensated;  // 1: TwoProd/TwoSum accumulation (pseudoinverse applies), 0: plain FMA
+  int compensated;  // 1: compensated accumulation (pseudoinverse applies: one segment, one group, A stays
+                    // put, no bscale, not accumulated, M and Kseg multiples of 8; needs sigma), 0: plain FMA
+  const double* sigma;  // compensated: start of every row's accumulation, cmp_sigma of its sum of |A|
   int mfma;         // plain form on the FP64 matrix cores (ignored when compensated):
                     // 2 wide tiles (up to 160 rows x 128 columns), 1 64 x 64 tiles, 0 VALU
   long ctot;        // all columns of the product (ncol x Rc)
@@ -132,6 +134,9 @@ struct GemmArgs {
   int bscale_seg;   // bscale applies to segments >= bscale_seg
 };
 void gemm(hipStream_t s, const GemmArgs& a);
+// Starting value of the compensated accumulation of a row of A: 1.5 2^m with
+// 2^(m - 2) at least the row's sum of |A|.
+double cmp_sigma(double abs_row_sum);
 // K splits the wide-tile product takes for these sizes (1: none).
 int gemm_split(const GemmArgs& a);
 

@@ -293,6 +293,15 @@ void Engine::upload_static()
   uc2ue_.upload(O.uc2ue);
   ue2uc_.upload(O.ue2uc);
   dc2de_.upload(O.dc2de);
+  // starting values of the compensated pseudoinverse applies, per operator row
+  auto sigma = [](const std::vector<double>& a, int m) {
+    std::vector<double> v(m, 0.0);
+    for (size_t k = 0; k < a.size(); k++) v[k % m] += std::fabs(a[k]);
+    for (double& x : v) x = dev::cmp_sigma(x);
+    return v;
+  };
+  uc2ue_sig_.upload(sigma(O.uc2ue, O.pln[SURF_UE]));
+  dc2de_sig_.upload(sigma(O.dc2de, O.pln[SURF_DE]));
   de2dc_.upload(O.de2dc);
   m2l_.upload(O.m2l);
   {  // frequency-major copies for the matrix-core M2L: [C][343][sdof][tdof] complex
@@ -342,12 +351,12 @@ void Engine::upload_static()
     dev::expand_m2l_vec(stream_, O.C, mm_.sdof, mm_.tdof, I_.p + plan_.aidx[1], opsT32_.p, avec32_.p);
   }
   {  // fused operator of the mixed up pass: m2me_ = UC2UE x [UE2UC_0 .. UE2UC_7],
-     // compensated (Dot2) like the pseudoinverse applies
+     // compensated like the pseudoinverse applies
     const int pUE = O.pln[SURF_UE], pUC = O.pln[SURF_UC];
     m2me_.alloc((size_t)8 * pUE * pUE);
     dev::GemmArgs a{};
     a.M = pUE; a.Kseg = pUC; a.nseg = 1; a.Rc = 1; a.ngroup = 1; a.maxcols = a.ncol = 8 * pUE;
-    a.A = uc2ue_.p; a.a_gstride = 0;
+    a.A = uc2ue_.p; a.a_gstride = 0; a.sigma = uc2ue_sig_.p;
     a.B = ue2uc_.p; a.bnode = I_.p + plan_.fuse_idx;
     a.C = m2me_.p; a.cnode = I_.p + plan_.fuse_idx; a.gbeg = I_.p + plan_.fuse_idx_g;
     a.compensated = 1;
@@ -364,7 +373,7 @@ void Engine::upload_static()
                             hipMemcpyDeviceToDevice, stream_));
     dev::GemmArgs a{};
     a.M = pDE; a.Kseg = pDC; a.nseg = 1; a.Rc = 1; a.ngroup = 1; a.maxcols = a.ncol = 8 * pDE;
-    a.A = dc2de_.p;
+    a.A = dc2de_.p; a.sigma = dc2de_sig_.p;
     a.B = de2dc_.p; a.bnode = I_.p + plan_.fdn_b;
     a.C = l2de_.p; a.cnode = I_.p + plan_.fdn_c; a.gbeg = I_.p + plan_.fdn_g;
     a.compensated = 1;
@@ -1354,6 +1363,7 @@ void Engine::run_chunk(const double* srcden, double* trgval, int rc, int mode, h
     a.cscale = op.cscale >= 0 ? D + op.cscale : nullptr;
     a.accumulate = op.accumulate;
     a.compensated = mixed ? 0 : op.compensated;
+    a.sigma = op.a_which == 0 ? uc2ue_sig_.p : dc2de_sig_.p;
     a.mfma = gemm_mfma_;
     a.ctot = (long)op.ncol * rc;
     a.work = gwork_.p;
