@@ -468,39 +468,83 @@ void scatter_rows(hipStream_t s, int n, int dof, int nr, const int* iperm, const
 constexpr int P2P_BS = 128;
 constexpr int TILE = 64;
 
-// The generic near-field kernels (k_p2p, k_p2p32) give one lane to each
-// target, except in a wave that holds at most 32 (16) of its chunk's
-// targets: there each target gets 2 (4) lanes, which take every second
-// (fourth) source, and sum() adds their partial sums into the first of them
-// (lanes l + 32 and l + 16 into lane l, in that order).  Near field per
-// evaluate: 1M Navier clusters 5.4 -> 4.5 ms (FP64), 2.8 -> 2.4 ms (FP32);
-// 262k Stokes sphere 0.95 -> 0.72 ms.  (The L2T / M2T kernel k_s2p measured
-// no gain from it.)  ON false (16-RHS blocks, whose register budget the
-// shuffled sums would overrun): one lane per target throughout.
-template <bool ON>
+// The FP64 vector near-field and L2T / M2T kernels (k_p2p, k_s2p) divide a block
+// of NF_BS threads into nsub = NF_BS / tn lanes per target of its chunk, which
+// take every nsub-th source of a staged tile; sum() adds their partial sums
+// through LDS in lane order, so the result does not depend on scheduling.  They
+// are bound by the FP64 vector rate where there are many chunks, and were by
+// latency otherwise: a leaf of an adaptive tree holds a few to a hundred
+// targets, so one lane per target left two thirds of a block idle (41 targets a
+// leaf on the 262k sphere) and gave each lane the chunk's whole list, several
+// thousand sources beside a refined region, as one serial chain.  Measured, with
+// tiles across entries (EntryList) and the plan's narrower chunks: near field
+// 3k Laplace 172 -> 24 us, 65k 388 -> 55 us, 262k Stokes sphere 689 -> 425 us,
+// 100k Stokeslets at 4 right-hand sides 1028 -> 331 us; L2T / M2T 967 -> 118 us
+// and 2489 -> 472 us on the last two, 1M Navier clusters 3730 -> 958 us.
+constexpr int NF_BS = 256;
+
 struct LaneSplit {
   int nsub, sub, ti;  // lanes per target, this lane's share, its target in the chunk
+  bool act;
   __device__ LaneSplit(int t, int tn)
   {
-    const int w = t >> 6, l = t & 63;
-    const int mw = min(64, max(0, tn - 64 * w));  // the wave's targets (wave-uniform)
-    nsub = !ON ? 1 : mw <= 16 ? 4 : mw <= 32 ? 2 : 1;
-    const int lpt = 64 / nsub;
-    ti = 64 * w + (l & (lpt - 1));
-    sub = l / lpt;
+    nsub = NF_BS / max(tn, 1);  // tn <= 128: at least 2
+    sub = t / max(tn, 1);
+    ti = t - sub * tn;
+    act = tn > 0 && sub < nsub;
   }
-  template <int A, int B>
-  __device__ void sum(double (&u)[A][B]) const
+  // val[q][d] += the sum over the lanes of a target; red: NF_BS * T doubles of
+  // LDS, free to use after a barrier
+  template <int NR, int T>
+  __device__ void sum(double (&u)[NR][T], double* red, int t, int tn, double* val, long val_rs) const
   {
-    if (!ON || nsub == 1) return;  // wave-uniform
 #pragma unroll
-    for (int a = 0; a < A; a++)
+    for (int q = 0; q < NR; q++) {
+      __syncthreads();
 #pragma unroll
-      for (int b = 0; b < B; b++) {
-        double v = u[a][b] + __shfl_down(u[a][b], 32);
-        if (nsub == 4) v += __shfl_down(v, 16);
-        u[a][b] = v;
+      for (int d = 0; d < T; d++) red[t * T + d] = u[q][d];
+      __syncthreads();
+      for (int i = t; i < tn * T; i += NF_BS) {
+        double v = red[i];
+        for (int s = 1; s < nsub; s++) v += red[s * tn * T + i];
+        val[(long)q * val_rs + i] += v;
       }
+    }
+  }
+};
+
+// The entries (source ranges) of a chunk as one list of sources, 64 entries at
+// a time: a staged tile takes its sources across entry boundaries, so leaves
+// of a few points fill whole tiles (65k uniform points in leaves of 16: 7
+// tiles and barrier pairs per chunk instead of 27).
+constexpr int EBATCH = 64;
+struct EntryList {
+  int off[EBATCH + 1];  // sources before each entry
+  int shift[EBATCH];    // source k of the batch is point k + shift of its entry
+  // wave 0 loads entries e0 .. e0 + n
+  __device__ void load(const int2* ent, int e0, int n, int t)
+  {
+    if (t >= EBATCH) return;
+    int2 se = make_int2(0, 0);
+    if (t < n) se = ent[e0 + t];
+    int in = se.y;
+#pragma unroll
+    for (int d = 1; d < 64; d *= 2) {
+      const int v = __shfl_up(in, d);
+      if (t >= d) in += v;
+    }
+    if (t == 0) off[0] = 0;
+    off[t + 1] = in;
+    shift[t] = se.x - (in - se.y);
+  }
+  __device__ int total() const { return off[EBATCH]; }
+  __device__ int point(int k) const
+  {
+    int i = 0;
+#pragma unroll
+    for (int d = EBATCH / 2; d > 0; d /= 2)
+      if (off[i + d] <= k) i += d;
+    return k + shift[i];
   }
 };
 
@@ -528,23 +572,29 @@ __device__ inline void stage_den(E (*s_den)[NR * S], const D* den, const Points&
   }
 }
 
+// FP64 near field on the vector units; densities from the FP64 copy or (src.den
+// null: the mixed form's pass over the entries its FP32 kernels skip) from the
+// FP32 one.
 template <int KT, int NR>
-__global__ __launch_bounds__(P2P_BS) void k_p2p(const int* __restrict__ tbeg, const int* __restrict__ tnum,
-                                                const int* __restrict__ eptr, const int2* __restrict__ ent, Points src,
-                                                Targets trg, int roff, KC kc)
+__global__ __launch_bounds__(NF_BS) void k_p2p(const int* __restrict__ tbeg, const int* __restrict__ tnum,
+                                               const int* __restrict__ eptr, const int2* __restrict__ ent, Points src,
+                                               Targets trg, int roff, KC kc)
 {
   using K = Knl<KT>;
-  constexpr int NPOS = K::NRM ? 6 : 3;
-  constexpr int ND = NR * K::S;
-  __shared__ double s_pos[TILE][NPOS];
-  __shared__ double s_den[TILE][ND];
+  constexpr int NPOS = K::NRM ? 6 : 3, ND = NR * K::S;
+  // sources per tile, by the LDS a row takes
+  constexpr int TW = ND <= 4 ? 256 : ND <= 12 ? 128 : 64;
+  __shared__ __align__(16) double lds[std::max(TW * (NPOS + ND), NF_BS * K::T)];
+  __shared__ EntryList s_ent;
+  __shared__ int s_pt[2][TW];
+  double(*const s_pos)[NPOS] = reinterpret_cast<double(*)[NPOS]>(lds);
+  double(*const s_den)[ND] = reinterpret_cast<double(*)[ND]>(lds + TW * NPOS);
   const int c = blockIdx.x, t = threadIdx.x;
   const int r0 = roff + blockIdx.y * NR;
   const int tb = tbeg[c], tn = tnum[c];
-  const LaneSplit<(NR < 16)> ls(t, tn);
-  const bool act = ls.ti < tn;
+  const LaneSplit ls(t, tn);
   double x = 0, y = 0, z = 0;
-  if (act) {
+  if (ls.act) {
     x = trg.x[tb + ls.ti];
     y = trg.y[tb + ls.ti];
     z = trg.z[tb + ls.ti];
@@ -554,77 +604,93 @@ __global__ __launch_bounds__(P2P_BS) void k_p2p(const int* __restrict__ tbeg, co
   for (int q = 0; q < NR; q++)
 #pragma unroll
     for (int d = 0; d < K::T; d++) u[q][d] = 0.0;
-  // FP64 densities, or (src.den null: the mixed form's pass over the entries
-  // its FP32 kernels skip) the FP32 copy
   const double* den = src.den ? src.den + (long)r0 * src.den_rs : nullptr;
   const float* den32 = src.den ? nullptr : src.den32 + (long)r0 * src.den_rs;
-  for (int e = eptr[c]; e < eptr[c + 1]; e++) {
-    const int2 se = ent[e];
-    for (int b0 = 0; b0 < se.y; b0 += TILE) {
-      const int cnt = min(TILE, se.y - b0);
-      const int j0 = se.x + b0;
+  const int e1 = eptr[c + 1];
+  for (int e0 = eptr[c]; e0 < e1; e0 += EBATCH) {
+    __syncthreads();
+    s_ent.load(ent, e0, min(EBATCH, e1 - e0), t);
+    __syncthreads();
+    const int total = s_ent.total();
+    // the points of a tile are looked up one tile ahead
+    if (t < min(TW, total)) s_pt[0][t] = s_ent.point(t);
+    for (int b0 = 0, buf = 0; b0 < total; b0 += TW, buf ^= 1) {
+      const int cnt = min(TW, total - b0);
       __syncthreads();
-      for (int i = t; i < cnt; i += P2P_BS) {
-        s_pos[i][0] = src.x[j0 + i];
-        s_pos[i][1] = src.y[j0 + i];
-        s_pos[i][2] = src.z[j0 + i];
+      for (int i = t; i < cnt; i += NF_BS) {
+        const int j = s_pt[buf][i];
+        s_pos[i][0] = src.x[j];
+        s_pos[i][1] = src.y[j];
+        s_pos[i][2] = src.z[j];
         if (K::NRM) {
-          s_pos[i][NPOS - 3] = src.nx[j0 + i];
-          s_pos[i][NPOS - 2] = src.ny[j0 + i];
-          s_pos[i][NPOS - 1] = src.nz[j0 + i];
+          s_pos[i][NPOS - 3] = src.nx[j];
+          s_pos[i][NPOS - 2] = src.ny[j];
+          s_pos[i][NPOS - 1] = src.nz[j];
         }
       }
+      auto stage = [&](auto* d) {
+        for (int i = t; i < cnt * ND; i += NF_BS) {
+          const int jj = i / ND, rem = i - jj * ND, q = rem / K::S;
+          s_den[jj][rem] = (double)d[(long)s_pt[buf][jj] * src.den_js + (long)q * src.den_rs + (rem - q * K::S)];
+        }
+      };
       if (den)
-        stage_den<K::S, NR, P2P_BS>(s_den, den, src, j0, cnt, t);
+        stage(den);
       else
-        stage_den<K::S, NR, P2P_BS>(s_den, den32, src, j0, cnt, t);
+        stage(den32);
+      if (t < min(TW, total - b0 - TW)) s_pt[buf ^ 1][t] = s_ent.point(b0 + TW + t);
       __syncthreads();
-      if (act)
+      if (ls.act)
+#pragma unroll 2
         for (int jj = ls.sub; jj < cnt; jj += ls.nsub)
           K::template add<NR>(x - s_pos[jj][0], y - s_pos[jj][1], z - s_pos[jj][2], &s_pos[jj][NPOS - 3], s_den[jj], u,
                               kc);
     }
   }
-  ls.sum(u);
-  if (act && ls.sub == 0) {
-    double* val = trg.val + (long)r0 * trg.val_rs + (long)(tb + ls.ti) * K::T;
-#pragma unroll
-    for (int q = 0; q < NR; q++)
-#pragma unroll
-      for (int d = 0; d < K::T; d++) val[(long)q * trg.val_rs + d] += u[q][d];
-  }
+  ls.sum(u, lds, t, tn, trg.val + (long)r0 * trg.val_rs + (long)tb * K::T, trg.val_rs);
 }
 
-// Mixed-precision form of k_p2p for the kernels without a matrix-core form:
-// coordinates relative to the chunk's first target computed in FP64 and
-// rounded, normals and densities rounded, the kernel evaluated in FP32 and the
-// sums of each staged tile (at most TILE sources) added in FP64.  Entries
-// flagged 2 in echk (a pair may be closer than the relative FP32 coordinates
-// resolve, so the r < 1e-8 rule needs the FP64 positions) are skipped: a
-// separate FP64 pass over those entries adds them.
+// Mixed-precision form of k_p2p for the kernels without normals: coordinates
+// relative to the chunk's first target computed in FP64 and rounded, densities
+// rounded, the kernel evaluated in FP32 and the sums of each tile (at most TILE
+// sources of one entry) added in FP64.  Entries flagged 2 in echk (a pair may
+// be closer than the relative FP32 coordinates resolve, so the r < 1e-8 rule
+// needs the FP64 positions) are skipped: a separate FP64 pass adds them.
+//
+// Every wave stages tiles of its own and shares none, so there is no barrier
+// per tile: the block's four waves take every fourth tile of the chunk (every
+// second for each half of a chunk of more than 64 targets), which shortens the
+// block's serial chain (1M Navier clusters 2.33 -> 2.17 ms).  In a wave that
+// holds at most 32 (16) targets a target has 2 (4) lanes, which take every
+// second (fourth) source of a tile.
 template <int KT, int NR>
-__global__ __launch_bounds__(P2P_BS) void k_p2p32(const int* __restrict__ tbeg, const int* __restrict__ tnum,
-                                                  const int* __restrict__ eptr, const int2* __restrict__ ent,
-                                                  const int* __restrict__ echk, Points src, Targets trg, int roff,
-                                                  KC kc)
+__global__ __launch_bounds__(NF_BS) void k_p2p32(const int* __restrict__ tbeg, const int* __restrict__ tnum,
+                                                 const int* __restrict__ eptr, const int2* __restrict__ ent,
+                                                 const int* __restrict__ echk, Points src, Targets trg, int roff,
+                                                 KC kc)
 {
   using K = Knl<KT>;
-  constexpr int NPOS = K::NRM ? 6 : 3;
-  constexpr int ND = NR * K::S;
-  __shared__ float s_pos[TILE][NPOS];
-  __shared__ float s_den[TILE][ND];
-  const int c = blockIdx.x, t = threadIdx.x;
+  static_assert(!K::NRM, "kernels with normals keep the FP64 near field");
+  constexpr int ND = NR * K::S, NW = NF_BS / 64, ROW = 3 + ND;
+  constexpr size_t LDS = std::max(sizeof(float) * NW * TILE * ROW, sizeof(double) * NF_BS * K::T);
+  __shared__ __align__(16) unsigned char lds[LDS];
+  __shared__ int s_off[EBATCH + 1], s_beg[EBATCH], s_num[EBATCH];
+  const int c = blockIdx.x, t = threadIdx.x, w = t >> 6, l = t & 63;
+  float(*const s_row)[ROW] = reinterpret_cast<float(*)[ROW]>(lds) + w * TILE;  // this wave's tile
   const int r0 = roff + blockIdx.y * NR;
   const int tb = tbeg[c], tn = tnum[c];
-  const LaneSplit<(NR < 16)> ls(t, tn);
-  const bool act = ls.ti < tn;
-  const int tb0 = tn > 0 ? tb : 0;  // origin of the relative coordinates
-  const double ox = trg.x[tb0], oy = trg.y[tb0], oz = trg.z[tb0];
+  const bool two = tn > 64;  // two halves of 64 targets
+  const int h = two ? w & 1 : 0, slot = two ? w >> 1 : w, nslot = two ? NW / 2 : NW;
+  const int mw = min(64, tn - 64 * h);  // the wave's targets
+  const int nsub = NR >= 16 ? 1 : mw <= 16 ? 4 : mw <= 32 ? 2 : 1, lpt = 64 / nsub;
+  const int sub = l / lpt, ti = 64 * h + (l & (lpt - 1));
+  const bool act = ti < tn;
+  const double ox = trg.x[tb], oy = trg.y[tb], oz = trg.z[tb];
   float x = 0, y = 0, z = 0;
   if (act) {
-    x = (float)(trg.x[tb + ls.ti] - ox);
-    y = (float)(trg.y[tb + ls.ti] - oy);
-    z = (float)(trg.z[tb + ls.ti] - oz);
+    x = (float)(trg.x[tb + ti] - ox);
+    y = (float)(trg.y[tb + ti] - oy);
+    z = (float)(trg.z[tb + ti] - oz);
   }
   double u[NR][K::T];
 #pragma unroll
@@ -632,48 +698,79 @@ __global__ __launch_bounds__(P2P_BS) void k_p2p32(const int* __restrict__ tbeg, 
 #pragma unroll
     for (int d = 0; d < K::T; d++) u[q][d] = 0.0;
   const double* den = src.den + (long)r0 * src.den_rs;
-  for (int e = eptr[c]; e < eptr[c + 1]; e++) {
-    if (echk && echk[e] == 2) continue;  // block-uniform: the FP64 pass's
-    const int2 se = ent[e];
-    for (int b0 = 0; b0 < se.y; b0 += TILE) {
-      const int cnt = min(TILE, se.y - b0);
-      const int j0 = se.x + b0;
-      __syncthreads();
-      for (int i = t; i < cnt; i += P2P_BS) {
-        s_pos[i][0] = (float)(src.x[j0 + i] - ox);
-        s_pos[i][1] = (float)(src.y[j0 + i] - oy);
-        s_pos[i][2] = (float)(src.z[j0 + i] - oz);
-        if (K::NRM) {
-          s_pos[i][NPOS - 3] = (float)src.nx[j0 + i];
-          s_pos[i][NPOS - 2] = (float)src.ny[j0 + i];
-          s_pos[i][NPOS - 1] = (float)src.nz[j0 + i];
-        }
+  const int e1 = eptr[c + 1];
+  for (int e0 = eptr[c]; e0 < e1; e0 += EBATCH) {
+    __syncthreads();
+    if (w == 0) {  // tiles before each of the next 64 entries
+      int2 se = make_int2(0, 0);
+      if (l < e1 - e0 && !(echk && echk[e0 + l] == 2)) se = ent[e0 + l];
+      int in = (se.y + TILE - 1) / TILE;
+#pragma unroll
+      for (int d = 1; d < 64; d *= 2) {
+        const int v = __shfl_up(in, d);
+        if (l >= d) in += v;
       }
-      stage_den<K::S, NR, P2P_BS>(s_den, den, src, j0, cnt, t);
-      __syncthreads();
-      if (act) {
-        float p[NR][K::T];
+      if (l == 0) s_off[0] = 0;
+      s_off[l + 1] = in;
+      s_beg[l] = se.x;
+      s_num[l] = se.y;
+    }
+    __syncthreads();
+    const int ntile = s_off[EBATCH];
+    for (int k = slot; k < ntile; k += nslot) {
+      int e = 0;
 #pragma unroll
-        for (int q = 0; q < NR; q++)
-#pragma unroll
-          for (int d = 0; d < K::T; d++) p[q][d] = 0.0f;
-        for (int jj = ls.sub; jj < cnt; jj += ls.nsub)
-          K::template add<NR>(x - s_pos[jj][0], y - s_pos[jj][1], z - s_pos[jj][2], &s_pos[jj][NPOS - 3], s_den[jj],
-                              p, kc);
-#pragma unroll
-        for (int q = 0; q < NR; q++)
-#pragma unroll
-          for (int d = 0; d < K::T; d++) u[q][d] += (double)p[q][d];
+      for (int d = EBATCH / 2; d > 0; d /= 2)
+        if (s_off[e + d] <= k) e += d;
+      const int b0 = (k - s_off[e]) * TILE, j0 = s_beg[e] + b0, cnt = min(TILE, s_num[e] - b0);
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // the previous tile has been read
+      __builtin_amdgcn_wave_barrier();
+      if (l < cnt) {
+        s_row[l][0] = (float)(src.x[j0 + l] - ox);
+        s_row[l][1] = (float)(src.y[j0 + l] - oy);
+        s_row[l][2] = (float)(src.z[j0 + l] - oz);
       }
+      for (int i = l; i < cnt * ND; i += 64) {
+        const int jj = i / ND, rem = i - jj * ND, q = rem / K::S;
+        s_row[jj][3 + rem] = (float)den[(long)(j0 + jj) * src.den_js + (long)q * src.den_rs + (rem - q * K::S)];
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      float p[NR][K::T];
+#pragma unroll
+      for (int q = 0; q < NR; q++)
+#pragma unroll
+        for (int d = 0; d < K::T; d++) p[q][d] = 0.0f;
+      if (act)
+        for (int jj = sub; jj < cnt; jj += nsub)
+          K::template add<NR>(x - s_row[jj][0], y - s_row[jj][1], z - s_row[jj][2], nullptr, &s_row[jj][3], p, kc);
+#pragma unroll
+      for (int q = 0; q < NR; q++)
+#pragma unroll
+        for (int d = 0; d < K::T; d++) u[q][d] += (double)p[q][d];
     }
   }
-  ls.sum(u);
-  if (act && ls.sub == 0) {
-    double* val = trg.val + (long)r0 * trg.val_rs + (long)(tb + ls.ti) * K::T;
+  // the lanes and waves of a target, in this order
+  double* const red = reinterpret_cast<double*>(lds);
+  double* const val = trg.val + (long)r0 * trg.val_rs + (long)tb * K::T;
 #pragma unroll
-    for (int q = 0; q < NR; q++)
+  for (int q = 0; q < NR; q++) {
+    __syncthreads();
 #pragma unroll
-      for (int d = 0; d < K::T; d++) val[(long)q * trg.val_rs + d] += u[q][d];
+    for (int d = 0; d < K::T; d++) {
+      double v = u[q][d];
+      if (nsub > 1) v += __shfl_down(v, 32);
+      if (nsub > 2) v += __shfl_down(v, 16);
+      red[t * K::T + d] = v;
+    }
+    __syncthreads();
+    if (slot == 0 && sub == 0 && act)
+#pragma unroll
+      for (int d = 0; d < K::T; d++) {
+        double v = red[t * K::T + d];
+        for (int o = 1; o < nslot; o++) v += red[(t + (NF_BS / nslot) * o) * K::T + d];
+        val[(long)q * trg.val_rs + (long)ti * K::T + d] += v;
+      }
   }
 }
 
@@ -739,6 +836,43 @@ __global__ __launch_bounds__(64) void k_p2p_s(const int* __restrict__ tbeg, cons
 typedef double v4d __attribute__((ext_vector_type(4)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 
+// The two waves of a matrix-core near-field block: 64 targets each, or, where
+// the chunk holds at most 64, the same targets in both, every second group of
+// 4 sources each, the second wave's sums added through LDS at the end (its
+// SIMD would idle, and the block's serial chain be twice as long).  FP64 only:
+// the FP32 kernels sum a whole tile in one FP32 chain.
+struct WaveSplit {
+  bool share;      // block-uniform
+  int base, ng;    // the wave's first target and its 16-target blocks
+  int g0, gs;      // its source groups of a tile
+  __device__ WaveSplit(int w, int tn, bool can_share = true)
+  {
+    share = can_share && tn <= 64;
+    base = share ? 0 : 64 * w;
+    ng = base < tn ? min(4, (tn - base + 15) >> 4) : 0;
+    g0 = share ? 4 * w : 0;
+    gs = share ? 8 : 4;
+  }
+  // acc of wave 0 += acc of wave 1; red: 1024 doubles of LDS, free after a barrier
+  template <class V>
+  __device__ void sum(V (&acc)[4], double* red, int w, int l) const
+  {
+    if (!share) return;
+    __syncthreads();
+    if (w == 1)
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int v = 0; v < 4; v++) red[(i * 4 + v) * 64 + l] = acc[i][v];
+    __syncthreads();
+    if (w == 0)
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int v = 0; v < 4; v++) acc[i][v] += red[(i * 4 + v) * 64 + l];
+  }
+};
+
 // One staged source tile against the wave's first NG 16-target column blocks
 // (NG = the blocks that hold targets, so ragged leaves do not pay for empty
 // blocks).
@@ -748,9 +882,9 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 template <int NG, bool GUARD = true>
 __device__ __forceinline__ void p2p_tile64(int cnt4, int kk, int col, const double (*s_pos)[TILE],
                                            const double (*s_den)[16], const double* tx, const double* ty,
-                                           const double* tz, v4d* acc)
+                                           const double* tz, v4d* acc, int g0 = 0, int gs = 4)
 {
-  for (int g = 0; g < cnt4; g += 4) {
+  for (int g = g0; g < cnt4; g += gs) {
     const double sx = s_pos[0][g + kk], sy = s_pos[1][g + kk], sz = s_pos[2][g + kk];
     const double f = s_den[g + kk][col];
 #pragma unroll
@@ -817,12 +951,12 @@ __global__ __launch_bounds__(P2P_BS) void k_p2p_mfma111(int nchunk, const int* _
   const int col = l & 15, kk = l >> 4;
   const int r0 = roff + blockIdx.y * NR;
   const int tb = tbeg[c], tn = tnum[c];
-  const bool wact = 64 * w < tn;  // wave-uniform
-  const int ng = wact ? min(4, (tn - 64 * w + 15) >> 4) : 0;  // 16-target blocks with targets
+  const WaveSplit ws(w, tn);
+  const int ng = ws.ng;  // wave-uniform
   double tx[4], ty[4], tz[4];
 #pragma unroll
   for (int i = 0; i < 4; i++) {
-    int tt = 64 * w + 16 * i + col;
+    int tt = ws.base + 16 * i + col;
     tt = tt < tn ? tt : 0;
     tx[i] = trg.x[tb + tt];
     ty[i] = trg.y[tb + tt];
@@ -850,27 +984,28 @@ __global__ __launch_bounds__(P2P_BS) void k_p2p_mfma111(int nchunk, const int* _
       __syncthreads();
       if (!guard) {
         if (ng == 4)
-          p2p_tile64<4, false>(cnt4, kk, col, s_pos, s_den, tx, ty, tz, acc);
+          p2p_tile64<4, false>(cnt4, kk, col, s_pos, s_den, tx, ty, tz, acc, ws.g0, ws.gs);
         else if (ng == 3)
-          p2p_tile64<3, false>(cnt4, kk, col, s_pos, s_den, tx, ty, tz, acc);
+          p2p_tile64<3, false>(cnt4, kk, col, s_pos, s_den, tx, ty, tz, acc, ws.g0, ws.gs);
         else if (ng == 2)
-          p2p_tile64<2, false>(cnt4, kk, col, s_pos, s_den, tx, ty, tz, acc);
+          p2p_tile64<2, false>(cnt4, kk, col, s_pos, s_den, tx, ty, tz, acc, ws.g0, ws.gs);
         else if (ng == 1)
-          p2p_tile64<1, false>(cnt4, kk, col, s_pos, s_den, tx, ty, tz, acc);
+          p2p_tile64<1, false>(cnt4, kk, col, s_pos, s_den, tx, ty, tz, acc, ws.g0, ws.gs);
       } else if (ng == 4)
-        p2p_tile64<4>(cnt4, kk, col, s_pos, s_den, tx, ty, tz, acc);
+        p2p_tile64<4>(cnt4, kk, col, s_pos, s_den, tx, ty, tz, acc, ws.g0, ws.gs);
       else if (ng == 3)
-        p2p_tile64<3>(cnt4, kk, col, s_pos, s_den, tx, ty, tz, acc);
+        p2p_tile64<3>(cnt4, kk, col, s_pos, s_den, tx, ty, tz, acc, ws.g0, ws.gs);
       else if (ng == 2)
-        p2p_tile64<2>(cnt4, kk, col, s_pos, s_den, tx, ty, tz, acc);
+        p2p_tile64<2>(cnt4, kk, col, s_pos, s_den, tx, ty, tz, acc, ws.g0, ws.gs);
       else if (ng == 1)
-        p2p_tile64<1>(cnt4, kk, col, s_pos, s_den, tx, ty, tz, acc);
+        p2p_tile64<1>(cnt4, kk, col, s_pos, s_den, tx, ty, tz, acc, ws.g0, ws.gs);
     }
   }
-  if (!wact) return;
+  ws.sum(acc, &s_den[0][0], w, l);
+  if (ws.share ? w > 0 : ng == 0) return;
 #pragma unroll
   for (int i = 0; i < 4; i++) {
-    const int tt = 64 * w + 16 * i + col;
+    const int tt = ws.base + 16 * i + col;
     if (tt < tn) {
       double* val = trg.val + (long)(r0 + kk) * trg.val_rs + tb + tt;
 #pragma unroll
@@ -902,13 +1037,13 @@ __global__ __launch_bounds__(P2P_BS) void k_p2p_mfma111_f32(int nchunk, const in
   const int col = l & 15, kk = l >> 4;
   const int r0 = roff + blockIdx.y * NR;
   const int tb = tbeg[c], tn = tnum[c];
-  const bool wact = 64 * w < tn;  // wave-uniform
-  const int ng = wact ? min(4, (tn - 64 * w + 15) >> 4) : 0;  // 16-target blocks with targets
+  const WaveSplit ws(w, tn, false);
+  const int ng = ws.ng;  // wave-uniform
   const double ox = trg.x[tb], oy = trg.y[tb], oz = trg.z[tb];
   float tx[4], ty[4], tz[4];
 #pragma unroll
   for (int i = 0; i < 4; i++) {
-    int tt = 64 * w + 16 * i + col;
+    int tt = ws.base + 16 * i + col;
     tt = tt < tn ? tt : 0;
     tx[i] = (float)(trg.x[tb + tt] - ox);
     ty[i] = (float)(trg.y[tb + tt] - oy);
@@ -986,10 +1121,10 @@ __global__ __launch_bounds__(P2P_BS) void k_p2p_mfma111_f32(int nchunk, const in
       }
     }
   }
-  if (!wact) return;
+  if (ng == 0) return;
 #pragma unroll
   for (int i = 0; i < 4; i++) {
-    const int tt = 64 * w + 16 * i + col;
+    const int tt = ws.base + 16 * i + col;
     if (tt < tn) {
       double* val = trg.val + (long)(r0 + 4 * kk) * trg.val_rs + tb + tt;
 #pragma unroll
@@ -1290,120 +1425,137 @@ __global__ __launch_bounds__(P2S_BS) void k_p2s(const int* __restrict__ out_node
 
 // ---------------------------------------------------------------------------
 // equivalent surface -> targets (L2T, M2T), mm kernel
+// The entries of a chunk (its own box, W boxes) are walked as one list of
+// surface points, as k_p2p walks its sources.
 template <int KT, int NR>
-__global__ __launch_bounds__(P2P_BS) void k_s2p(const int* __restrict__ tbeg, const int* __restrict__ tnum,
-                                                const int* __restrict__ eptr, const int* __restrict__ enode,
-                                                const int* __restrict__ ekind, const double4* __restrict__ egeom,
-                                                const double* __restrict__ unit_de, const double* __restrict__ unit_ue,
-                                                int nsp, const double* __restrict__ dneden,
-                                                const double* __restrict__ upeden, int Rc, int pln, Targets trg,
-                                                int roff, KC kc)
+__global__ __launch_bounds__(NF_BS) void k_s2p(const int* __restrict__ tbeg, const int* __restrict__ tnum,
+                                               const int* __restrict__ eptr, const int* __restrict__ enode,
+                                               const int* __restrict__ ekind, const double4* __restrict__ egeom,
+                                               const double* __restrict__ unit_de, const double* __restrict__ unit_ue,
+                                               int nsp, const double* __restrict__ dneden,
+                                               const double* __restrict__ upeden, int Rc, int pln, Targets trg,
+                                               int roff, KC kc)
 {
   using K = Knl<KT>;
   constexpr int ND = NR * K::S;
-  __shared__ double s_pos[TILE][3];
-  __shared__ double s_den[TILE][ND];
+  constexpr int TW = ND <= 4 ? 256 : ND <= 16 ? 128 : 64;
+  constexpr size_t LDS = sizeof(double) * std::max(TW * (3 + ND), NF_BS * K::T);
+  __shared__ __align__(16) unsigned char lds[LDS];
+  __shared__ long s_at[TW];  // where a source's densities start in dneden, or ~ of it in upeden
+  double(*const s_pos)[3] = reinterpret_cast<double(*)[3]>(lds);
+  double(*const s_den)[ND] = reinterpret_cast<double(*)[ND]>(lds + sizeof(double) * TW * 3);
   const int c = blockIdx.x, t = threadIdx.x;
   const int r0 = roff + blockIdx.y * NR;
   const int tb = tbeg[c], tn = tnum[c];
-  const bool act = t < tn;
+  const LaneSplit ls(t, tn);
   double x = 0, y = 0, z = 0;
-  if (act) {
-    x = trg.x[tb + t];
-    y = trg.y[tb + t];
-    z = trg.z[tb + t];
+  if (ls.act) {
+    x = trg.x[tb + ls.ti];
+    y = trg.y[tb + ls.ti];
+    z = trg.z[tb + ls.ti];
   }
   double u[NR][K::T];
 #pragma unroll
   for (int q = 0; q < NR; q++)
 #pragma unroll
     for (int d = 0; d < K::T; d++) u[q][d] = 0.0;
-  for (int e = eptr[c]; e < eptr[c + 1]; e++) {
-    const int kind = ekind[e];
-    const double* unit = kind == 0 ? unit_de : unit_ue;
-    const double* buf = (kind == 0 ? dneden : upeden) + ((long)enode[e] * Rc + r0) * pln;
-    const double4 g = egeom[e];
-    for (int b0 = 0; b0 < nsp; b0 += TILE) {
-      const int cnt = min(TILE, nsp - b0);
-      __syncthreads();
-      for (int i = t; i < cnt; i += P2P_BS) {
-        s_pos[i][0] = g.x + g.w * unit[3 * (b0 + i)];
-        s_pos[i][1] = g.y + g.w * unit[3 * (b0 + i) + 1];
-        s_pos[i][2] = g.z + g.w * unit[3 * (b0 + i) + 2];
-      }
-      const int per = cnt * K::S;
-      for (int i = t; i < NR * per; i += P2P_BS) {
-        int q = i / per, rem = i - q * per;
-        int jj = rem / K::S, sd = rem - jj * K::S;
-        s_den[jj][q * K::S + sd] = buf[(long)q * pln + (long)b0 * K::S + rem];
-      }
-      __syncthreads();
-      if (act)
-        for (int jj = 0; jj < cnt; jj++)
-          K::template add<NR>(x - s_pos[jj][0], y - s_pos[jj][1], z - s_pos[jj][2], nullptr, s_den[jj], u, kc);
+  const int e0 = eptr[c];
+  const long total = (long)(eptr[c + 1] - e0) * nsp;
+  for (long b0 = 0; b0 < total; b0 += TW) {
+    const int cnt = (int)min((long)TW, total - b0);
+    __syncthreads();
+    if (t < cnt) {
+      const int e = e0 + (int)((b0 + t) / nsp), pt = (int)(b0 + t - (long)(e - e0) * nsp);
+      const bool de = ekind[e] == 0;
+      const double* unit = (de ? unit_de : unit_ue) + 3 * pt;
+      const double4 g = egeom[e];
+      const long at = ((long)enode[e] * Rc + r0) * pln + (long)pt * K::S;
+      s_at[t] = de ? at : ~at;
+      s_pos[t][0] = g.x + g.w * unit[0];
+      s_pos[t][1] = g.y + g.w * unit[1];
+      s_pos[t][2] = g.z + g.w * unit[2];
     }
-  }
-  if (act) {
-    double* val = trg.val + (long)r0 * trg.val_rs + (long)(tb + t) * K::T;
-#pragma unroll
+    __syncthreads();
+    const int per = cnt * K::S;
     for (int q = 0; q < NR; q++)
-#pragma unroll
-      for (int d = 0; d < K::T; d++) val[(long)q * trg.val_rs + d] += u[q][d];
+      for (int i = t; i < per; i += NF_BS) {
+        const int jj = i / K::S, d = i - jj * K::S;
+        const long at = s_at[jj];
+        s_den[jj][q * K::S + d] = (at >= 0 ? dneden[at + (long)q * pln + d] : upeden[~at + (long)q * pln + d]);
+      }
+    __syncthreads();
+    if (ls.act)
+#pragma unroll 2
+      for (int jj = ls.sub; jj < cnt; jj += ls.nsub)
+        K::template add<NR>(x - s_pos[jj][0], y - s_pos[jj][1], z - s_pos[jj][2], nullptr, s_den[jj], u, kc);
   }
+  ls.sum(u, reinterpret_cast<double*>(lds), t, tn, trg.val + (long)r0 * trg.val_rs + (long)tb * K::T, trg.val_rs);
 }
 
 template <int KT, int NR>
-static void p2p_launch(hipStream_t s, int variant, int nchunk, int nb, const int* tbeg, const int* tnum,
-                       const int* eptr, const int2* ent, const int* echk, Points src, Targets trg, int roff, KC kc)
+static void p2p_launch(hipStream_t s, int variant, const Near& c, int nb, Points src, Targets trg, int roff, KC kc)
 {
   if (variant >= 2 && KT == 111 && NR == 16 && src.den_rs == 1)
-    hipLaunchKernelGGL(k_p2p_mfma111, dim3(xcd_grid(nchunk), nb), dim3(P2P_BS), 0, s, nchunk, tbeg, tnum, eptr, ent,
-                       echk, src, trg, roff, kc);
+    hipLaunchKernelGGL(k_p2p_mfma111, dim3(xcd_grid(c.n), nb), dim3(P2P_BS), 0, s, c.n, c.tbeg, c.tnum, c.eptr, c.ent,
+                       c.chk, src, trg, roff, kc);
   else if (variant == 1)
-    hipLaunchKernelGGL((k_p2p_s<KT, NR>), dim3(2 * nchunk, nb), dim3(64), 0, s, tbeg, tnum, eptr, ent, src, trg, roff,
-                       kc);
-  else if (variant == 4)
-    hipLaunchKernelGGL((k_p2p32<KT, NR>), dim3(nchunk, nb), dim3(P2P_BS), 0, s, tbeg, tnum, eptr, ent, echk, src, trg,
+    hipLaunchKernelGGL((k_p2p_s<KT, NR>), dim3(2 * c.n, nb), dim3(64), 0, s, c.tbeg, c.tnum, c.eptr, c.ent, src, trg,
                        roff, kc);
   else
-    hipLaunchKernelGGL((k_p2p<KT, NR>), dim3(nchunk, nb), dim3(P2P_BS), 0, s, tbeg, tnum, eptr, ent, src, trg, roff,
-                       kc);
+    hipLaunchKernelGGL((k_p2p<KT, NR>), dim3(c.n, nb), dim3(NF_BS), 0, s, c.tbeg, c.tnum, c.eptr, c.ent, src, trg,
+                       roff, kc);
 }
 
 template <int KT>
-static int p2p_kt(hipStream_t s, int nchunk, const int* tbeg, const int* tnum, const int* eptr, const int2* ent,
-                  const int* echk, Points src, Targets trg, int nr, KC kc, int variant)
+static void p2p_kt(hipStream_t s, const Near& c, Points src, Targets trg, int r0, int nr, KC kc, int variant)
 {
-  int r0 = 0;
-  if (KT == 111 && variant == 3 && echk) {
-    const int left = rhs_blocks16(nr, [&](int nb, int roff, int nrv) {
-      hipLaunchKernelGGL(k_p2p_mfma111_f32, dim3(xcd_grid(nchunk), nb), dim3(P2P_BS), 0, s, nchunk, tbeg, tnum, eptr,
-                         ent, echk, src, trg, roff, kc, nrv);
-    });
-    r0 = nr - left;
-  }
   rhs_blocks(nr - r0, [&](int NR, int nb, int roff) {
     if (NR == 16)
-      p2p_launch<KT, 16>(s, variant, nchunk, nb, tbeg, tnum, eptr, ent, echk, src, trg, r0 + roff, kc);
+      p2p_launch<KT, 16>(s, variant, c, nb, src, trg, r0 + roff, kc);
     else if (NR == 4)
-      p2p_launch<KT, 4>(s, variant, nchunk, nb, tbeg, tnum, eptr, ent, echk, src, trg, r0 + roff, kc);
+      p2p_launch<KT, 4>(s, variant, c, nb, src, trg, r0 + roff, kc);
     else
-      p2p_launch<KT, 1>(s, variant, nchunk, nb, tbeg, tnum, eptr, ent, echk, src, trg, r0 + roff, kc);
+      p2p_launch<KT, 1>(s, variant, c, nb, src, trg, r0 + roff, kc);
   });
-  // right-hand sides [0, n) went through a kernel that skips flagged entries
-  return variant == 4 && echk ? nr : r0;
 }
 
-int p2p(hipStream_t s, int kt, int nchunk, const int* tbeg, const int* tnum, const int* eptr, const int2* ent,
-        const int* echk, Points src, Targets trg, int nr, KC kc, int variant)
+void p2p(hipStream_t s, int kt, const Near& c, Points src, Targets trg, int r0, int nr, KC kc, int variant)
 {
-  if (nchunk <= 0) return 0;
+  if (c.n <= 0) return;
   switch (kt) {
 #define KIFMM_P2P(KT) \
-  case KT: return p2p_kt<KT>(s, nchunk, tbeg, tnum, eptr, ent, echk, src, trg, nr, kc, variant);
+  case KT: p2p_kt<KT>(s, c, src, trg, r0, nr, kc, variant); break;
   KIFMM_P2P(111) KIFMM_P2P(121) KIFMM_P2P(311) KIFMM_P2P(312) KIFMM_P2P(321) KIFMM_P2P(322) KIFMM_P2P(511)
   KIFMM_P2P(521)
 #undef KIFMM_P2P
+  }
+}
+
+template <int KT>
+static void p2p32_kt(hipStream_t s, const Near& c, Points src, Targets trg, int nr, KC kc)
+{
+  rhs_blocks(nr, [&](int NR, int nb, int roff) {
+    const dim3 grid(c.n, nb), bs(NF_BS);
+    if (NR == 16)
+      hipLaunchKernelGGL((k_p2p32<KT, 16>), grid, bs, 0, s, c.tbeg, c.tnum, c.eptr, c.ent, c.chk, src, trg, roff, kc);
+    else if (NR == 4)
+      hipLaunchKernelGGL((k_p2p32<KT, 4>), grid, bs, 0, s, c.tbeg, c.tnum, c.eptr, c.ent, c.chk, src, trg, roff, kc);
+    else
+      hipLaunchKernelGGL((k_p2p32<KT, 1>), grid, bs, 0, s, c.tbeg, c.tnum, c.eptr, c.ent, c.chk, src, trg, roff, kc);
+  });
+}
+
+int p2p32(hipStream_t s, int kt, const Near& c, Points src, Targets trg, int nr, KC kc)
+{
+  if (c.n <= 0) return nr;
+  switch (kt) {
+  case 111:
+    return nr - rhs_blocks16(nr, [&](int nb, int roff, int nrv) {
+      hipLaunchKernelGGL(k_p2p_mfma111_f32, dim3(xcd_grid(c.n), nb), dim3(P2P_BS), 0, s, c.n, c.tbeg, c.tnum, c.eptr,
+                         c.ent, c.chk, src, trg, roff, kc, nrv);
+    });
+  case 311: p2p32_kt<311>(s, c, src, trg, nr, kc); return nr;
+  case 511: p2p32_kt<511>(s, c, src, trg, nr, kc); return nr;
   }
   return 0;
 }
@@ -1679,20 +1831,20 @@ __global__ __launch_bounds__(P2P_BS) void k_s2p_mfma111(int nchunk, const int* _
   // FP32: 160 surface points per staged tile, all of an np 6 surface (152) in one
   constexpr int NR = 16, TL = F32 ? S2P_TILE32 : TILE;
   __shared__ R s_pos[3][TL];
-  __shared__ R s_den[TL][NR];
+  __shared__ __align__(16) R s_den[TL][NR];
   const int c = xcd_item(blockIdx.x, nchunk), t = threadIdx.x, w = t >> 6, l = t & 63;
   if (c >= nchunk) return;  // block-uniform
   const int col = l & 15, kk = l >> 4;
   const int r0 = roff + blockIdx.y * NR;
   const int tb = tbeg[c], tn = tnum[c];
-  const bool wact = 64 * w < tn;  // wave-uniform
-  const int ng = wact ? min(4, (tn - 64 * w + 15) >> 4) : 0;
+  const WaveSplit ws(w, tn, !F32);
+  const int ng = ws.ng;  // wave-uniform
   // FP32: coordinates relative to the chunk's first target; FP64: absolute
   const double ox = F32 ? trg.x[tb] : 0.0, oy = F32 ? trg.y[tb] : 0.0, oz = F32 ? trg.z[tb] : 0.0;
   R tx[4], ty[4], tz[4];
 #pragma unroll
   for (int i = 0; i < 4; i++) {
-    int tt = 64 * w + 16 * i + col;
+    int tt = ws.base + 16 * i + col;
     tt = tt < tn ? tt : 0;
     tx[i] = (R)(trg.x[tb + tt] - ox);
     ty[i] = (R)(trg.y[tb + tt] - oy);
@@ -1742,23 +1894,24 @@ __global__ __launch_bounds__(P2P_BS) void k_s2p_mfma111(int nchunk, const int* _
       } else {
         if (ng == 4)
           p2p_tile64<4>(cnt4, kk, col, (const double(*)[TILE])s_pos, (const double(*)[16])s_den, (const double*)tx,
-                        (const double*)ty, (const double*)tz, accm);
+                        (const double*)ty, (const double*)tz, accm, ws.g0, ws.gs);
         else if (ng == 3)
           p2p_tile64<3>(cnt4, kk, col, (const double(*)[TILE])s_pos, (const double(*)[16])s_den, (const double*)tx,
-                        (const double*)ty, (const double*)tz, accm);
+                        (const double*)ty, (const double*)tz, accm, ws.g0, ws.gs);
         else if (ng == 2)
           p2p_tile64<2>(cnt4, kk, col, (const double(*)[TILE])s_pos, (const double(*)[16])s_den, (const double*)tx,
-                        (const double*)ty, (const double*)tz, accm);
+                        (const double*)ty, (const double*)tz, accm, ws.g0, ws.gs);
         else if (ng == 1)
           p2p_tile64<1>(cnt4, kk, col, (const double(*)[TILE])s_pos, (const double(*)[16])s_den, (const double*)tx,
-                        (const double*)ty, (const double*)tz, accm);
+                        (const double*)ty, (const double*)tz, accm, ws.g0, ws.gs);
       }
     }
   }
-  if (!wact) return;
+  if constexpr (!F32) ws.sum(accm, &s_den[0][0], w, l);
+  if (ws.share ? w > 0 : ng == 0) return;
 #pragma unroll
   for (int i = 0; i < 4; i++) {
-    const int tt = 64 * w + 16 * i + col;
+    const int tt = ws.base + 16 * i + col;
     if (tt >= tn) continue;
     if constexpr (F32) {  // FP32 item v of lane l: right-hand side 4*(l/16) + v
       double* val = trg.val + (long)(r0 + 4 * kk) * trg.val_rs + tb + tt;
@@ -1775,54 +1928,46 @@ __global__ __launch_bounds__(P2P_BS) void k_s2p_mfma111(int nchunk, const int* _
 }
 
 template <int KT>
-static void s2p_kt(hipStream_t s, int nchunk, const int* tbeg, const int* tnum, const int* eptr, const int* enode,
-                   const int* ekind, const double4* egeom, const double* unit_de, const double* unit_ue, int nsp,
+static void s2p_kt(hipStream_t s, const Far& wide, const Far& c, const double* unit_de, const double* unit_ue, int nsp,
                    const double* dneden, const double* upeden, int Rc, int pln, Targets trg, int nr, KC kc,
                    int variant)
 {
   int r0 = 0;
   if (KT == 111 && variant == 3) {
     r0 = nr - rhs_blocks16(nr, [&](int nb, int roff, int nrv) {
-      hipLaunchKernelGGL((k_s2p_mfma111<true>), dim3(xcd_grid(nchunk), nb), dim3(P2P_BS), 0, s, nchunk, tbeg, tnum,
-                         eptr, enode, ekind, egeom, unit_de, unit_ue, nsp, dneden, upeden, Rc, pln, trg, roff, kc, nrv);
+      hipLaunchKernelGGL((k_s2p_mfma111<true>), dim3(xcd_grid(wide.n), nb), dim3(P2P_BS), 0, s, wide.n, wide.tbeg,
+                         wide.tnum, wide.eptr, wide.node, wide.kind, wide.geom, unit_de, unit_ue, nsp, dneden, upeden,
+                         Rc, pln, trg, roff, kc, nrv);
     });
   }
   rhs_blocks(nr - r0, [&](int NR, int nb, int roff0) {
     const int roff = r0 + roff0;
-    dim3 grid(nchunk, nb);
+    const dim3 grid(c.n, nb), bs(NF_BS);
     if (KT == 111 && NR == 16 && variant == 2)
-      hipLaunchKernelGGL((k_s2p_mfma111<false>), dim3(xcd_grid(nchunk), nb), dim3(P2P_BS), 0, s, nchunk, tbeg, tnum,
-                         eptr, enode, ekind, egeom, unit_de, unit_ue, nsp, dneden, upeden, Rc, pln, trg, roff, kc, 16);
+      hipLaunchKernelGGL((k_s2p_mfma111<false>), dim3(xcd_grid(c.n), nb), dim3(P2P_BS), 0, s, c.n, c.tbeg, c.tnum,
+                         c.eptr, c.node, c.kind, c.geom, unit_de, unit_ue, nsp, dneden, upeden, Rc, pln, trg, roff, kc,
+                         16);
     else if (NR == 16)
-      hipLaunchKernelGGL((k_s2p<KT, 16>), grid, dim3(P2P_BS), 0, s, tbeg, tnum, eptr, enode, ekind, egeom, unit_de,
+      hipLaunchKernelGGL((k_s2p<KT, 16>), grid, bs, 0, s, c.tbeg, c.tnum, c.eptr, c.node, c.kind, c.geom, unit_de,
                          unit_ue, nsp, dneden, upeden, Rc, pln, trg, roff, kc);
     else if (NR == 4)
-      hipLaunchKernelGGL((k_s2p<KT, 4>), grid, dim3(P2P_BS), 0, s, tbeg, tnum, eptr, enode, ekind, egeom, unit_de,
+      hipLaunchKernelGGL((k_s2p<KT, 4>), grid, bs, 0, s, c.tbeg, c.tnum, c.eptr, c.node, c.kind, c.geom, unit_de,
                          unit_ue, nsp, dneden, upeden, Rc, pln, trg, roff, kc);
     else
-      hipLaunchKernelGGL((k_s2p<KT, 1>), grid, dim3(P2P_BS), 0, s, tbeg, tnum, eptr, enode, ekind, egeom, unit_de,
+      hipLaunchKernelGGL((k_s2p<KT, 1>), grid, bs, 0, s, c.tbeg, c.tnum, c.eptr, c.node, c.kind, c.geom, unit_de,
                          unit_ue, nsp, dneden, upeden, Rc, pln, trg, roff, kc);
   });
 }
 
-void s2p(hipStream_t s, int kt, int nchunk, const int* tbeg, const int* tnum, const int* eptr, const int* enode,
-         const int* ekind, const double4* egeom, const double* unit_de, const double* unit_ue, int nsp,
+void s2p(hipStream_t s, int kt, const Far& wide, const Far& c, const double* unit_de, const double* unit_ue, int nsp,
          const double* dneden, const double* upeden, int Rc, int pln, Targets trg, int nr, KC kc, int variant)
 {
-  if (nchunk <= 0) return;
+  if (c.n <= 0) return;
   switch (kt) {
-  case 111:
-    s2p_kt<111>(s, nchunk, tbeg, tnum, eptr, enode, ekind, egeom, unit_de, unit_ue, nsp, dneden, upeden, Rc, pln, trg,
-                nr, kc, variant);
-    break;
-  case 301:
-    s2p_kt<301>(s, nchunk, tbeg, tnum, eptr, enode, ekind, egeom, unit_de, unit_ue, nsp, dneden, upeden, Rc, pln, trg,
-                nr, kc, variant);
-    break;
-  case 511:
-    s2p_kt<511>(s, nchunk, tbeg, tnum, eptr, enode, ekind, egeom, unit_de, unit_ue, nsp, dneden, upeden, Rc, pln, trg,
-                nr, kc, variant);
-    break;
+#define KIFMM_S2P(KT) \
+  case KT: s2p_kt<KT>(s, wide, c, unit_de, unit_ue, nsp, dneden, upeden, Rc, pln, trg, nr, kc, variant); break;
+  KIFMM_S2P(111) KIFMM_S2P(301) KIFMM_S2P(511)
+#undef KIFMM_S2P
   }
 }
 

@@ -58,23 +58,29 @@ struct Targets {  // leaf-ordered targets (SoA) and values [rhs][n*tdof]
   long val_rs;
 };
 
-// Near field: for every chunk of <= 128 targets, sum the user kernel over the
-// source leaves ent[eptr[c] .. eptr[c+1]) (each ent = {sextbeg, sextnum}).
-// variant 0: sources staged in LDS, 128-thread blocks; variant 1: sources read
-// through the scalar cache (needs den_rs == sdof), one wave per 64 targets;
-// variant 2: Laplace blocks of 16 right-hand sides on the FP64 matrix cores;
-// variant 3: the same on the FP32 matrix cores (mixed precision).  Variants
-// 2 and 3 fall back to variant 0 for other kernels and smaller blocks.
-// variant 4: the kernels without normals in FP32 (mixed precision).
-// echk[e] (variants 2, 3 and 4; without it variant 3 takes the FP64
-// matrix-core kernel): 0 no pair of entry e can be closer than 1e-8 or than
-// its FP32 offsets resolve (the FP64 matrix-core kernel skips the exclusion
-// test there), 1 the target's own leaf (exclusion tested), 2 a pair may be
-// closer than the FP32 offsets resolve: the FP32 kernels skip such entries.  Returns n: right-hand sides [0, n) skipped the entries flagged 2,
-// which a second call with variant 0 over those entries alone (and nr = n)
-// then adds in FP64.
-int p2p(hipStream_t s, int kt, int nchunk, const int* tbeg, const int* tnum, const int* eptr, const int2* ent,
-        const int* echk, Points src, Targets trg, int nr, KC kc, int variant);
+// Chunks of <= 128 targets of one leaf (targets [tbeg[c], tbeg[c] + tnum[c])).
+// Near field: entries [eptr[c], eptr[c+1]), each a source range {sextbeg,
+// sextnum}, and how the r < 1e-8 exclusion applies to its pairs: chk[e] 0 no
+// pair can be closer than 1e-8 or than its FP32 offsets resolve (the FP64
+// matrix-core kernel skips the exclusion test there), 1 the target's own leaf
+// (exclusion tested), 2 a pair may be closer than the FP32 offsets resolve.
+struct Near {
+  int n;
+  const int *tbeg, *tnum, *eptr;
+  const int2* ent;
+  const int* chk;
+};
+// FP64 near field of right-hand sides [r0, nr): the user kernel summed over
+// every chunk's sources.  variant 0: sources staged in LDS; 1: sources read
+// through the scalar cache (needs den_rs == sdof), one wave per 64 targets; 2
+// and 3: Laplace blocks of 16 right-hand sides on the FP64 matrix cores, other
+// kernels and smaller blocks as variant 0.
+void p2p(hipStream_t s, int kt, const Near& c, Points src, Targets trg, int r0, int nr, KC kc, int variant);
+// FP32 near field (mixed precision): Laplace blocks of 16 right-hand sides on
+// the FP32 matrix cores, the kernels without normals on the vector units.
+// Returns n: right-hand sides [0, n) are done but for the entries flagged 2,
+// which p2p over those entries alone then adds in FP64.
+int p2p32(hipStream_t s, int kt, const Near& c, Points src, Targets trg, int nr, KC kc);
 
 // Set-up pass for the mixed near field, per entry e of the near-field chunks:
 // out[e].x = the smallest squared distance between a chunk target and an
@@ -97,12 +103,16 @@ void p2s(hipStream_t s, int kt, int nitem, const int* out_node, const double4* g
          int variant, int accum = 1);
 
 // Equivalent surfaces to targets with the mm kernel (L2T from DE, M2T from UE).
-// Entry e: node enode[e] of buffer ekind[e] (0 = dneden, 1 = upeden), surface
-// ekind 0 -> unit_de, 1 -> unit_ue, placed at geom[e] = (cx, cy, cz, rad).
+// Entry e of a chunk: node[e] of buffer kind[e] (0 = dneden, 1 = upeden), surface
+// kind 0 -> unit_de, 1 -> unit_ue, placed at geom[e] = (cx, cy, cz, rad).
 // variant (Laplace, 16-RHS blocks): 2 FP64 matrix cores, 3 FP32 matrix cores
-// (mixed form), otherwise the FP64 vector kernels.
-void s2p(hipStream_t s, int kt, int nchunk, const int* tbeg, const int* tnum, const int* eptr, const int* enode,
-         const int* ekind, const double4* egeom, const double* unit_de, const double* unit_ue, int nsp,
+// (mixed form, over the chunks `wide`), otherwise the FP64 vector kernels.
+struct Far {
+  int n;
+  const int *tbeg, *tnum, *eptr, *node, *kind;
+  const double4* geom;
+};
+void s2p(hipStream_t s, int kt, const Far& wide, const Far& c, const double* unit_de, const double* unit_ue, int nsp,
          const double* dneden, const double* upeden, int Rc, int pln, Targets trg, int nr, KC kc, int variant);
 
 // Batched, indexed FP64 GEMM over (node, rhs) columns:

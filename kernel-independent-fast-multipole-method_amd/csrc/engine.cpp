@@ -277,6 +277,13 @@ void Engine::near_flags()
                  nent);
   if (nent) HIPCHK(hipMemcpy(I_.p + P.near.chk, chk.data(), sizeof(int) * nent, hipMemcpyHostToDevice));
   std::copy(chk.begin(), chk.end(), P.I.begin() + P.near.chk);
+  if (!P.near_wide.empty()) {  // the FP64 kernels' narrower chunks take the flags of theirs
+    std::vector<int> c64;
+    for (int w : P.near_wide) c64.insert(c64.end(), chk.begin() + eptr[w], chk.begin() + eptr[w + 1]);
+    if (!c64.empty())
+      HIPCHK(hipMemcpy(I_.p + P.near64.chk, c64.data(), sizeof(int) * c64.size(), hipMemcpyHostToDevice));
+    std::copy(c64.begin(), c64.end(), P.I.begin() + P.near64.chk);
+  }
   if (ftb.empty()) return;
   P.near_fix.n = (int)ftb.size();
   P.near_fix.tbeg = pool_i(F, ftb);
@@ -498,13 +505,18 @@ void Engine::build_plan()
   }
   // near field, S2L items and L2T/M2T chunks, per target leaf
   {
-    std::vector<int> tbeg, tnum, eptr(1, 0), ent, echk;
-    std::vector<int> ftbeg, ftnum, feptr(1, 0), fnode, fkind;
-    std::vector<double> fgeom;
     std::vector<int> xout, xeptr(1, 0), xent;
     std::vector<double> xgeom;
     std::vector<int> dent, dchk, sent, sknd;
     std::vector<double> sgeom;
+    struct Leaf {
+      int g;
+      long nlist, flist;  // sources and surface points of its near and far entries
+      int nd, ns;         // these entries
+    };
+    std::vector<Leaf> leaves;
+    std::vector<int> lent, lchk, lnode, lkind;
+    std::vector<double> lgeom;
     for (int g = 0; g < T.nnode; g++) {
       if (!(T.tag[g] & NODE_TRG)) continue;
       const bool leaf = T.terminal(g);
@@ -556,26 +568,78 @@ void Engine::build_plan()
       }
       P.near_pairs += npair * T.textnum[g];
       P.far_pairs += fpair * T.textnum[g];
-      for (int off = 0; off < T.textnum[g]; off += 128) {
-        int n = std::min(128, T.textnum[g] - off);
-        tbeg.push_back(T.textbeg[g] + off); tnum.push_back(n);
-        ent.insert(ent.end(), dent.begin(), dent.end());
-        echk.insert(echk.end(), dchk.begin(), dchk.end());
-        eptr.push_back((int)ent.size() / 2);
-        ftbeg.push_back(T.textbeg[g] + off); ftnum.push_back(n);
-        fnode.insert(fnode.end(), sent.begin(), sent.end());
-        fkind.insert(fkind.end(), sknd.begin(), sknd.end());
-        fgeom.insert(fgeom.end(), sgeom.begin(), sgeom.end());
-        feptr.push_back((int)fnode.size());
-      }
+      leaves.push_back({g, npair, fpair, (int)dchk.size(), (int)sknd.size()});
+      lent.insert(lent.end(), dent.begin(), dent.end());
+      lchk.insert(lchk.end(), dchk.begin(), dchk.end());
+      lnode.insert(lnode.end(), sent.begin(), sent.end());
+      lkind.insert(lkind.end(), sknd.begin(), sknd.end());
+      lgeom.insert(lgeom.end(), sgeom.begin(), sgeom.end());
     }
-    P.near.n = (int)tbeg.size();
-    P.near.tbeg = pool_i(P.I, tbeg); P.near.tnum = pool_i(P.I, tnum);
-    P.near.eptr = pool_i(P.I, eptr); P.near.ent = pool_i(P.I, ent); P.near.chk = pool_i(P.I, echk);
-    P.far.n = (int)ftbeg.size();
-    P.far.tbeg = pool_i(P.I, ftbeg); P.far.tnum = pool_i(P.I, ftnum);
-    P.far.eptr = pool_i(P.I, feptr); P.far.enode = pool_i(P.I, fnode);
-    P.far.ekind = pool_i(P.I, fkind); P.far.egeom = pool_d(P.D, fgeom);
+    // Chunks of up to 128 targets of a leaf; a second set, for the FP64 kernels,
+    // has fewer where the leaf's list is much longer than the others' (a coarse
+    // leaf beside a refined region lists up to 95 boxes of 152 surface points,
+    // the mean being 3): a block shares a chunk's pairs among its 256 threads,
+    // so halving the chunk halves its serial chain.  A chain may take 512 pairs
+    // or a quarter of the vector units' mean share of all pairs (1024 SIMDs of
+    // 64 lanes), whichever is more: below either a longer chain does not show.
+    // The FP32 kernels keep the first set: their coordinates are relative to
+    // the chunk's first target.
+    auto chain_limit = [](long pairs) { return std::max(512L, pairs / (4 * 1024 * 64)); };
+    const long nlim = chain_limit(P.near_pairs), flim = chain_limit(P.far_pairs);
+    auto width = [](long list, long lim) {
+      int w = 128;
+      while (w > 16 && list * w / 256 > lim) w /= 2;
+      return w;
+    };
+    auto chunks = [&](bool narrow) {
+      std::vector<int> tbeg, tnum, eptr(1, 0), ent, echk;
+      std::vector<int> ftbeg, ftnum, feptr(1, 0), fnode, fkind;
+      std::vector<double> fgeom;
+      ChunkList near, far;
+      size_t d0 = 0, s0 = 0;
+      int wide0 = 0;  // the leaf's first chunk of the first set
+      for (const Leaf& l : leaves) {
+        const int nt = T.textnum[l.g], tb = T.textbeg[l.g];
+        const int wn = narrow ? width(l.nlist, nlim) : 128, wf = narrow ? width(l.flist, flim) : 128;
+        for (int off = 0; off < nt; off += wn) {
+          tbeg.push_back(tb + off); tnum.push_back(std::min(wn, nt - off));
+          ent.insert(ent.end(), lent.begin() + 2 * d0, lent.begin() + 2 * (d0 + l.nd));
+          echk.insert(echk.end(), lchk.begin() + d0, lchk.begin() + d0 + l.nd);
+          eptr.push_back((int)ent.size() / 2);
+          if (narrow) P.near_wide.push_back(wide0 + off / 128);
+        }
+        for (int off = 0; off < nt; off += wf) {
+          ftbeg.push_back(tb + off); ftnum.push_back(std::min(wf, nt - off));
+          fnode.insert(fnode.end(), lnode.begin() + s0, lnode.begin() + s0 + l.ns);
+          fkind.insert(fkind.end(), lkind.begin() + s0, lkind.begin() + s0 + l.ns);
+          fgeom.insert(fgeom.end(), lgeom.begin() + 4 * s0, lgeom.begin() + 4 * (s0 + l.ns));
+          feptr.push_back((int)fnode.size());
+        }
+        d0 += l.nd;
+        s0 += l.ns;
+        wide0 += (nt + 127) / 128;
+      }
+      near.n = (int)tbeg.size();
+      far.n = (int)ftbeg.size();
+      if (!narrow || near.n != P.near.n) {
+        near.tbeg = pool_i(P.I, tbeg); near.tnum = pool_i(P.I, tnum);
+        near.eptr = pool_i(P.I, eptr); near.ent = pool_i(P.I, ent); near.chk = pool_i(P.I, echk);
+      } else {  // no leaf was cut
+        near = P.near;
+        P.near_wide.clear();
+      }
+      if (!narrow || far.n != P.far.n) {
+        far.tbeg = pool_i(P.I, ftbeg); far.tnum = pool_i(P.I, ftnum);
+        far.eptr = pool_i(P.I, feptr); far.enode = pool_i(P.I, fnode);
+        far.ekind = pool_i(P.I, fkind); far.egeom = pool_d(P.D, fgeom);
+      } else {
+        far = P.far;
+      }
+      (narrow ? P.near64 : P.near) = near;
+      (narrow ? P.far64 : P.far) = far;
+    };
+    chunks(false);
+    chunks(true);
     P.s2l.n = (int)xout.size();
     P.s2l.out = pool_i(P.I, xout); P.s2l.eptr = pool_i(P.I, xeptr);
     P.s2l.ent = pool_i(P.I, xent); P.s2l.geom = pool_d(P.D, xgeom);
@@ -1432,14 +1496,16 @@ void Engine::run_chunk(const double* srcden, double* trgval, int rc, int mode, h
     HIPCHK(hipStreamWaitEvent(side_, fork_ev_, 0));
   }
   timed_on(side ? side_ : s, KIFMM3D_K_P2P, [&] {
-    const int n32 = dev::p2p(side ? side_ : s, user_.kt, P.near.n, I + P.near.tbeg, I + P.near.tnum,
-                             I + P.near.eptr, (const int2*)(I + P.near.ent), I + P.near.chk, src, trg, rc, kcu, nvar);
+    const hipStream_t ns = side ? side_ : s;
+    const auto near = [](const int* I, const ChunkList& l) {
+      return dev::Near{l.n, I + l.tbeg, I + l.tnum, I + l.eptr, (const int2*)(I + l.ent), I + l.chk};
+    };
+    const int n32 = nvar == 3 || nvar == 4 ? dev::p2p32(ns, user_.kt, near(I, P.near), src, trg, rc, kcu) : 0;
+    dev::p2p(ns, user_.kt, near(I, P.near64), src, trg, n32, rc, kcu, nvar);
     if (near_fix && n32 > 0) {
-      const int* F = fix_.p;
       dev::Points sfix = src;
       sfix.den = den64;  // null when only the FP32 copy was gathered
-      dev::p2p(side ? side_ : s, user_.kt, P.near_fix.n, F + P.near_fix.tbeg, F + P.near_fix.tnum,
-               F + P.near_fix.eptr, (const int2*)(F + P.near_fix.ent), nullptr, sfix, trg, n32, kcu, 0);
+      dev::p2p(ns, user_.kt, near(fix_.p, P.near_fix), sfix, trg, 0, n32, kcu, 0);
     }
   });
   if (side) HIPCHK(hipEventRecord(join_ev_, side_));
@@ -1502,8 +1568,10 @@ void Engine::run_chunk(const double* srcden, double* trgval, int rc, int mode, h
   if (side) HIPCHK(hipStreamWaitEvent(s, join_ev_, 0));
   // L2T + M2T
   timed(KIFMM3D_K_S2P, [&] {
-    dev::s2p(s, mm_.kt, P.far.n, I + P.far.tbeg, I + P.far.tnum, I + P.far.eptr, I + P.far.enode,
-             I + P.far.ekind, (const double4*)(D + P.far.egeom), unit_[SURF_DE].p, unit_[SURF_UE].p,
+    const auto far = [&](const ChunkList& l) {
+      return dev::Far{l.n, I + l.tbeg, I + l.tnum, I + l.eptr, I + l.enode, I + l.ekind, (const double4*)(D + l.egeom)};
+    };
+    dev::s2p(s, mm_.kt, far(P.far), far(P.far64), unit_[SURF_DE].p, unit_[SURF_UE].p,
              O.nsp[SURF_DE], dneden_.p, upeden_.p, rc, pDE, trg, rc, kcm, mixed ? 3 : p2p_variant_);
   });
   mark(7);

@@ -76,6 +76,8 @@ struct VLevel {
 struct Plan {
   ItemList s2m, s2l;
   ChunkList near, far;
+  ChunkList near64, far64;     // the FP64 kernels': narrower where a leaf's list is long
+  std::vector<int> near_wide;  // near chunk that each near64 chunk is part of (empty: the same list)
   // the near-field chunks that hold entries flagged 2 (chk), with only those
   // entries (offsets into the engine's fix_ pool, set at the device set-up):
   // the FP32 near fields skip them and this FP64 pass adds them
