@@ -2642,8 +2642,9 @@ void gemm(hipStream_t s, const GemmArgs& a)
 // inverse evaluates only the surface points.
 //
 // Spectra are stored per slot either right-hand-side major ([slot][r][f][C],
-// rhs_inner = 0) or right-hand-side innermost ([slot][f][C][Rc], rhs_inner =
-// 1, the layout of the tiled matrix-core M2L); CT is double2 or float2.
+// SPEC_FREQ_INNER), right-hand-side innermost ([slot][f][C][Rc], the layout of
+// the tiled matrix-core M2L) or dof innermost ([slot][Rc][C][f], that of the
+// parent-grouped one); CT is double2 or float2.
 
 // Arithmetic of the transforms: FP64 for FP64 spectra, FP32 for FP32 spectra
 // (the spectra are rounded to FP32 for the M2L products either way).
@@ -2731,11 +2732,27 @@ __device__ __forceinline__ void fft_half_in(A2 lo, A2 hi, A2& s, A2& d)
   d.y = lo.y - hi.y;
 }
 
-template <int NP, class CT>
+// Strides of a spectrum value over right-hand sides, dofs and frequencies.
+struct SpecStride {
+  long r, d, f;
+};
+static SpecStride spec_stride(int layout, int C, int Rc, int dof)
+{
+  if (layout == SPEC_RHS_INNER) return {1, (long)C * Rc, Rc};
+  if (layout == SPEC_DOF_INNER) return {(long)dof * C, 1, dof};
+  return {(long)dof * C, C, 1};
+}
+
+// A block transforms one right-hand side of a slot, FD of its dofs at a time:
+// the z stage of all of them together writes the dof-innermost spectra as whole
+// lines (a dof at a time, 16 of every 64 bytes, the Stokes sphere's forward
+// transforms took 410 us, 186 with frequencies innermost).
+template <int NP, class CT, int FD>
 __global__ __launch_bounds__(256) void k_fft_fwd(const int* __restrict__ slot_node, int Rc,
                                                  const double* __restrict__ upeden, int pln, int sm,
                                                  const double* __restrict__ dscale, const short* __restrict__ c2s,
-                                                 CT* __restrict__ effden, const double2* __restrict__ tw, int rhs_inner)
+                                                 CT* __restrict__ effden, const double2* __restrict__ tw,
+                                                 SpecStride st)
 {
   constexpr int N = 2 * NP, H = NP + 1, C = N * N * H, NC = NP * NP * NP;
   constexpr int NSP = NP * NP * NP - (NP - 2) * (NP - 2) * (NP - 2);
@@ -2745,56 +2762,58 @@ __global__ __launch_bounds__(256) void k_fft_fwd(const int* __restrict__ slot_no
   __shared__ short s_c2s[NC];
   __shared__ A2 s_w[N];
   __shared__ A2 X1[NP * NP * H];
-  __shared__ A2 X2[NP * N * H];
+  __shared__ A2 X2[FD][NP * N * H];
   const int slot = blockIdx.x, r = blockIdx.y, t = threadIdx.x;
   const double* den = upeden + ((long)slot_node[slot] * Rc + r) * pln;
   for (int i = t; i < pln; i += 256) s_den[i] = (A)(den[i] * dscale[i % sm]);
   for (int i = t; i < NC; i += 256) s_c2s[i] = c2s[i];
   if (t < N) s_w[t] = cget<A2>(tw[t]);
   __syncthreads();
-  const long os = rhs_inner ? Rc : 1;
-  CT* out = effden + (long)slot * Rc * sm * C + (rhs_inner ? (long)r : (long)r * sm * C);
-  for (int f = 0; f < sm; f++) {
-    for (int o = t; o < NP * NP * H; o += 256) {  // along x: X1[k][j][kx]
-      int kx = o % H, j = (o / H) % NP, k = o / (H * NP);
-      A2 acc = cz<A2>();
+  CT* out = effden + (long)slot * Rc * sm * C + r * st.r;
+  for (int fa = 0; fa < sm; fa += FD) {  // FD divides sm
+#pragma unroll 1
+    for (int f = fa; f < fa + FD; f++) {
+      for (int o = t; o < NP * NP * H; o += 256) {  // along x: X1[k][j][kx]
+        int kx = o % H, j = (o / H) % NP, k = o / (H * NP);
+        A2 acc = cz<A2>();
 #pragma unroll
-      for (int i = 0; i < NP; i++) {
-        int si = s_c2s[(i * NP + j) * NP + k];
-        if (si >= 0) {
-          const A v = s_den[si * sm + f];
-          const A2 w = s_w[((i + NP / 2) * kx) % N];
-          acc.x += v * w.x;
-          acc.y += v * w.y;
+        for (int i = 0; i < NP; i++) {
+          int si = s_c2s[(i * NP + j) * NP + k];
+          if (si >= 0) {
+            const A v = s_den[si * sm + f];
+            const A2 w = s_w[((i + NP / 2) * kx) % N];
+            acc.x += v * w.x;
+            acc.y += v * w.y;
+          }
         }
+        X1[o] = acc;
       }
-      X1[o] = acc;
-    }
-    __syncthreads();
-    for (int o = t; o < NP * N * H; o += 256) {  // along y: X2[k][ky][kx]
-      int kx = o % H, ky = (o / H) % N, k = o / (H * N);
-      A2 acc = cz<A2>();
+      __syncthreads();
+      for (int o = t; o < NP * N * H; o += 256) {  // along y: X2[k][ky][kx]
+        int kx = o % H, ky = (o / H) % N, k = o / (H * N);
+        A2 acc = cz<A2>();
 #pragma unroll
-      for (int j = 0; j < NP; j++) {
-        const A2 v = cmul2(X1[(k * NP + j) * H + kx], s_w[((j + NP / 2) * ky) % N]);
-        acc.x += v.x;
-        acc.y += v.y;
+        for (int j = 0; j < NP; j++) {
+          const A2 v = cmul2(X1[(k * NP + j) * H + kx], s_w[((j + NP / 2) * ky) % N]);
+          acc.x += v.x;
+          acc.y += v.y;
+        }
+        X2[f - fa][o] = acc;
       }
-      X2[o] = acc;
+      __syncthreads();
     }
-    __syncthreads();
-    for (int o = t; o < C; o += 256) {  // along z
+    for (int e = t; e < C * FD; e += 256) {  // along z, in the order of the stores
+      const int d = st.d == 1 ? e % FD : e / C, o = st.d == 1 ? e / FD : e - d * C;
       int kx = o % H, ky = (o / H) % N, kz = o / (H * N);
       A2 acc = cz<A2>();
 #pragma unroll
       for (int k = 0; k < NP; k++) {
-        const A2 v = cmul2(X2[(k * N + ky) * H + kx], s_w[((k + NP / 2) * kz) % N]);
+        const A2 v = cmul2(X2[d][(k * N + ky) * H + kx], s_w[((k + NP / 2) * kz) % N]);
         acc.x += v.x;
         acc.y += v.y;
       }
-      cset(out[((long)f * C + o) * os], acc);
+      cset(out[(fa + d) * st.d + o * st.f], acc);
     }
-    __syncthreads();
   }
 }
 
@@ -2802,7 +2821,7 @@ template <int NP, class CT>
 __global__ __launch_bounds__(256) void k_fft_inv(const int* __restrict__ slot_node, int Rc,
                                                  const CT* __restrict__ effval, int tm,
                                                  const int* __restrict__ s2c, int nsp, double* __restrict__ dncval,
-                                                 int pln, const double2* __restrict__ tw, int rhs_inner)
+                                                 int pln, const double2* __restrict__ tw, SpecStride st)
 {
   constexpr int N = 2 * NP, H = NP + 1, C = N * N * H;
   using A = typename FftMath<CT>::A;
@@ -2813,11 +2832,10 @@ __global__ __launch_bounds__(256) void k_fft_inv(const int* __restrict__ slot_no
   const int slot = blockIdx.x, r = blockIdx.y, t = threadIdx.x;
   if (t < N) s_w[t] = cget<A2>(tw[t]);
   double* out = dncval + ((long)slot_node[slot] * Rc + r) * pln;
-  const long os = rhs_inner ? Rc : 1;
-  const CT* in = effval + (long)slot * Rc * tm * C + (rhs_inner ? (long)r : (long)r * tm * C);
+  const CT* in = effval + (long)slot * Rc * tm * C + r * st.r;
   for (int f = 0; f < tm; f++) {
     __syncthreads();
-    for (int o = t; o < C; o += 256) s_x[o] = cget<A2>(in[((long)f * C + o) * os]);
+    for (int o = t; o < C; o += 256) s_x[o] = cget<A2>(in[f * st.d + o * st.f]);
     __syncthreads();
     for (int o = t; o < NP * N * H; o += 256) {  // along z, only the cube's planes
       int kx = o % H, ky = (o / H) % N, k = o / (H * N);
@@ -3130,10 +3148,11 @@ constexpr int FFT_RW32_FWD = 8, FFT_RW32_INV = 8;
 
 template <class CT>
 static void fft_fwd_t(hipStream_t s, int np, int nslot, const int* slot_node, int Rc, const double* upeden, int pln,
-                      int sm, const double* dscale, const short* cube2surf, CT* effden, const double2* tw, int ri)
+                      int sm, const double* dscale, const short* cube2surf, CT* effden, const double2* tw,
+                      int layout)
 {
   if (nslot <= 0) return;
-  if (ri && sm == 1) {
+  if (layout == SPEC_RHS_INNER && sm == 1) {
     constexpr int RW = sizeof(CT) == 8 ? FFT_RW32_FWD : 4;
     // np 6: the x and y stages fused, a block writing whole 128-byte lines
     // of spectra: 16 FP32 right-hand sides (1024 threads) or 8 FP64 ones
@@ -3154,20 +3173,35 @@ static void fft_fwd_t(hipStream_t s, int np, int nslot, const int* slot_node, in
     }
     return;
   }
-  dim3 grid(nslot, Rc);
+  const SpecStride st = spec_stride(layout, 2 * np * 2 * np * (np + 1), Rc, sm);
+  // all dofs at once but for 4 of np 8 in FP64 (92 KB of LDS, one block per CU)
+  const dim3 grid(nslot, Rc);
+  auto go = [&](auto npc, auto fdc) {
+    hipLaunchKernelGGL((k_fft_fwd<npc, CT, fdc>), grid, dim3(256), 0, s, slot_node, Rc, upeden, pln, sm, dscale,
+                       cube2surf, effden, tw, st);
+  };
+  auto by_sm = [&](auto npc) {
+    constexpr int FD4 = npc == 8 && sizeof(CT) == 16 ? 1 : 4;
+    if (sm == 4)
+      go(npc, std::integral_constant<int, FD4>{});
+    else if (sm == 3)
+      go(npc, std::integral_constant<int, 3>{});
+    else
+      go(npc, std::integral_constant<int, 1>{});
+  };
   switch (np) {
-  case 4: hipLaunchKernelGGL((k_fft_fwd<4, CT>), grid, dim3(256), 0, s, slot_node, Rc, upeden, pln, sm, dscale, cube2surf, effden, tw, ri); break;
-  case 6: hipLaunchKernelGGL((k_fft_fwd<6, CT>), grid, dim3(256), 0, s, slot_node, Rc, upeden, pln, sm, dscale, cube2surf, effden, tw, ri); break;
-  case 8: hipLaunchKernelGGL((k_fft_fwd<8, CT>), grid, dim3(256), 0, s, slot_node, Rc, upeden, pln, sm, dscale, cube2surf, effden, tw, ri); break;
+  case 4: by_sm(std::integral_constant<int, 4>{}); break;
+  case 6: by_sm(std::integral_constant<int, 6>{}); break;
+  case 8: by_sm(std::integral_constant<int, 8>{}); break;
   }
 }
 
 template <class CT>
 static void fft_inv_t(hipStream_t s, int np, int nslot, const int* slot_node, int Rc, const CT* effval, int tm,
-                      const int* surf2cube, int nsp, double* dncval, int pln, const double2* tw, int ri)
+                      const int* surf2cube, int nsp, double* dncval, int pln, const double2* tw, int layout)
 {
   if (nslot <= 0) return;
-  if (ri && tm == 1) {
+  if (layout == SPEC_RHS_INNER && tm == 1) {
     constexpr int RW = sizeof(CT) == 8 ? FFT_RW32_INV : 4;
     // np 6, FP64: 6 waves for the 4 right-hand sides of a block, so the z
     // stage's 336 lines take one pass and 3 blocks fit a CU (4M points /
@@ -3186,30 +3220,31 @@ static void fft_inv_t(hipStream_t s, int np, int nslot, const int* slot_node, in
     }
     return;
   }
+  const SpecStride st = spec_stride(layout, 2 * np * 2 * np * (np + 1), Rc, tm);
   dim3 grid(nslot, Rc);
   switch (np) {
-  case 4: hipLaunchKernelGGL((k_fft_inv<4, CT>), grid, dim3(256), 0, s, slot_node, Rc, effval, tm, surf2cube, nsp, dncval, pln, tw, ri); break;
-  case 6: hipLaunchKernelGGL((k_fft_inv<6, CT>), grid, dim3(256), 0, s, slot_node, Rc, effval, tm, surf2cube, nsp, dncval, pln, tw, ri); break;
-  case 8: hipLaunchKernelGGL((k_fft_inv<8, CT>), grid, dim3(256), 0, s, slot_node, Rc, effval, tm, surf2cube, nsp, dncval, pln, tw, ri); break;
+  case 4: hipLaunchKernelGGL((k_fft_inv<4, CT>), grid, dim3(256), 0, s, slot_node, Rc, effval, tm, surf2cube, nsp, dncval, pln, tw, st); break;
+  case 6: hipLaunchKernelGGL((k_fft_inv<6, CT>), grid, dim3(256), 0, s, slot_node, Rc, effval, tm, surf2cube, nsp, dncval, pln, tw, st); break;
+  case 8: hipLaunchKernelGGL((k_fft_inv<8, CT>), grid, dim3(256), 0, s, slot_node, Rc, effval, tm, surf2cube, nsp, dncval, pln, tw, st); break;
   }
 }
 
 void fft_fwd(hipStream_t s, int np, int nslot, const int* slot_node, int Rc, const double* upeden, int pln, int sm,
-             const double* dscale, const short* cube2surf, void* effden, int single, int rhs_inner, const double2* tw)
+             const double* dscale, const short* cube2surf, void* effden, int single, int layout, const double2* tw)
 {
   if (single)
-    fft_fwd_t(s, np, nslot, slot_node, Rc, upeden, pln, sm, dscale, cube2surf, (float2*)effden, tw, rhs_inner);
+    fft_fwd_t(s, np, nslot, slot_node, Rc, upeden, pln, sm, dscale, cube2surf, (float2*)effden, tw, layout);
   else
-    fft_fwd_t(s, np, nslot, slot_node, Rc, upeden, pln, sm, dscale, cube2surf, (double2*)effden, tw, rhs_inner);
+    fft_fwd_t(s, np, nslot, slot_node, Rc, upeden, pln, sm, dscale, cube2surf, (double2*)effden, tw, layout);
 }
 
 void fft_inv(hipStream_t s, int np, int nslot, const int* slot_node, int Rc, const void* effval, int single,
-             int rhs_inner, int tm, const int* surf2cube, int nsp, double* dncval, int pln, const double2* tw)
+             int layout, int tm, const int* surf2cube, int nsp, double* dncval, int pln, const double2* tw)
 {
   if (single)
-    fft_inv_t(s, np, nslot, slot_node, Rc, (const float2*)effval, tm, surf2cube, nsp, dncval, pln, tw, rhs_inner);
+    fft_inv_t(s, np, nslot, slot_node, Rc, (const float2*)effval, tm, surf2cube, nsp, dncval, pln, tw, layout);
   else
-    fft_inv_t(s, np, nslot, slot_node, Rc, (const double2*)effval, tm, surf2cube, nsp, dncval, pln, tw, rhs_inner);
+    fft_inv_t(s, np, nslot, slot_node, Rc, (const double2*)effval, tm, surf2cube, nsp, dncval, pln, tw, layout);
 }
 
 // ---------------------------------------------------------------------------
@@ -3953,46 +3988,44 @@ void m2l_wave(hipStream_t s, int C, int ntile, int Rc, int nslot, const int* tti
 
 // ---------------------------------------------------------------------------
 // M2L on the matrix cores for any kernel and any number of right-hand sides
-// (spectra in the [slot][rhs][dof][C] layout of the grouped plan).
+// (spectra in the [slot][rhs][C][dof] layout).
 //
 // For one frequency f and neighbour direction n, the M2L of a target parent
 // T is the complex product Y_T[(c,t)] += sum_{(s,j)} M_n[(c,t)][(s,j)]
 // X_{T+n}[(s,j)] over the 8 TM outputs (child c, dof t) and the 8 SM inputs
-// (source child s, dof j), M_n[(c,t)][(s,j)] = T_{optab[n][s][c]}[j][t](f).
+// (source child s, dof j), M_n[(c,t)][(s,j)] = T_o[j][t](f) with the offset
+// o = 2 n + s - c, zero where the children are adjacent (|o|_inf < 2).
 // M_n does not depend on T, so the product is batched over columns =
 // (target parent, right-hand side) pairs, 16 per matrix-core tile, in real form
 //   [Yr; Yi] += [[Mr, -Mi], [Mi, Mr]] [Xr; Xi]
-// with v_mfma_f64_16x16x4f64.  Row tile rt < TM holds 16 real rows: row r16
-// is output rt*8 + r16%8 (flattened (c, t)), real part for r16 < 8.  The 16 SM
-// real inputs are cut into 4 SM slices of 4; input kappa is part kappa/(8 SM)
-// of flattened (s, j) = kappa % (8 SM).  With the output layout of the
-// instruction (item v of lane l is row l/16 + 4v) lane (k, col) ends with
-// (re, im) of outputs rt*8 + k and rt*8 + k + 4.
+// with v_mfma_f64_16x16x4f64.  Row tile rt < TM holds 16 real rows: output
+// rt*8 + row_out(r16) (flattened (c, t)), real or imaginary part (Mv).  The 16
+// SM real inputs are cut into 4 SM slices of 4; input kappa is part
+// kappa/(8 SM) of flattened (s, j) = kappa % (8 SM).
 //
-// A block covers FB consecutive frequencies and 4 tiles of 16 columns (one
-// per wave).  For each direction the block builds [[Mr,-Mi],[Mi,Mr]] of each
-// frequency in LDS from the frequency-major operator copy opsT [C][343][SM][TM]
-// through a frequency-independent index table, and every wave applies them to
-// its tile; a lane loads the FB frequencies of each source spectrum as one
-// contiguous run.  pmask[q] has bit n set if
-// parent q has a source child in direction n; a tile whose parents have none
-// skips the direction.  The blocks of one column block and 8 neighbouring
-// frequencies are dealt to one XCD side by side, so each 128-byte line of
-// spectra (8 frequencies) is fetched into its L2 once for all 8.
+// Operators.  The 64 child pairs of a direction share the 27 operators of the
+// offsets 2 n + d, d = s - c in {-1, 0, 1}^3, so a block keeps only those in
+// LDS, as three planes (Mr, Mi, -Mi) of [27][t][j] values, and a lane reads
+// its A operand at lane base (c, t, row part) + offset (s, j): none of it
+// depends on n, and each of a direction's values is loaded once, coalesced.
+// (Expanded to [[Mr, -Mi], [Mi, Mr]] per direction, the 4 tdof sdof x 64 entries
+// cost as much to gather as the products to form, and the FP32 form read them
+// from a table of up to 552 MB.)  M2L per evaluate: 262k Stokes sphere FP64 4.75
+// -> 3.47 ms, FP32 2.41 -> 2.25 ms; 1M Navier clusters FP32 17.4 -> 13.4 ms; 100k
+// Stokeslets at 4 right-hand sides 5.76 -> 4.03 ms.
+// The planes are double-buffered: one barrier per direction, the next
+// direction's operators and source slots in flight while one is applied.
+//
+// Columns.  The dofs of a frequency and the FB consecutive frequencies of the
+// block are contiguous, so the 4 lanes of a column read whole lines of a
+// source spectrum instead of 16 bytes of a line each.  A tile skips what none
+// of its columns has: a direction, or a source child (slice) of it.
+//
+// DS = 1: 4 tiles of 16 columns per block, one per wave, sharing the operators.
+// DS = 4, for levels with too few blocks to fill the chip: one tile, wave w
+// taking the directions n = w mod 4 with operators of its own, the partial sums
+// added through LDS in wave order; 7 rounds instead of 26 serial directions.
 constexpr int M2LV_BS = 256;
-
-// Raw buffer loads (gfx9 resource word 3; offsets past the resource's size
-// read zeros).
-constexpr int BUF_DW3 = 0x00020000;
-template <class R> __device__ inline R buf_ld(__amdgpu_buffer_rsrc_t r, unsigned off, int soff);
-template <> __device__ inline float buf_ld<float>(__amdgpu_buffer_rsrc_t r, unsigned off, int soff)
-{
-  return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, off, soff, 0));
-}
-template <> __device__ inline double buf_ld<double>(__amdgpu_buffer_rsrc_t r, unsigned off, int soff)
-{
-  return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, off, soff, 0));
-}
 
 // Precision traits of the parent-grouped M2L.  FP64: row r16 of a row tile is
 // output r16 % 8, part r16 / 8, so accumulator items (h, h + 2) of lane k are
@@ -4024,35 +4057,25 @@ struct Mv<float> {
   __device__ static inline int item_im(int h) { return 2 * h + 1; }
 };
 
-// The loads of a direction are issued before its barriers: the operator-
-// table entries and source slots of direction n + 1 are loaded while
-// direction n is applied, and the operator values (through a buffer resource:
-// one 32-bit offset per entry for both frequencies) and the source spectra of
-// a direction are fetched together, so a direction waits on one memory round
-// trip instead of four.  Measured against the direction-by-direction order
-// (1M Navier clusters, 262k Stokes sphere, M2L per evaluate): FP64 3x3 29.0 ->
-// 26.7 ms, FP64 4x3 5.4 -> 4.7 ms, FP32 4x3 3.5 -> 2.9 ms, FP32 3x3 19.8 ->
-// 19.9 ms.
-//
-// XA: the A operands come from the table expanded at set-up (atabv, [C][26]
-// [NA] in the block's entry order, signs and zeros applied), one coalesced
-// run per (frequency, direction), instead of gathers through aidx from the
-// operators (1M Navier clusters, FP32: M2L 19.9 -> 16.8 ms).
-template <class R, int SM, int TM, int FB, bool XA>
+template <class R, int SM, int TM, int FB, int DS>
 __global__ __launch_bounds__(M2LV_BS) void k_m2l_vec(int C, int Rc, long ncol, int ncb, const int* __restrict__ tslot,
                                                      const int* __restrict__ sslot, const int* __restrict__ pmask,
-                                                     const int* __restrict__ aidx,
                                                      const typename Mv<R>::C2* __restrict__ opsT,
-                                                     const R* __restrict__ atabv,
                                                      const typename Mv<R>::C2* __restrict__ effden,
                                                      typename Mv<R>::C2* __restrict__ effval)
 {
   typedef typename Mv<R>::C2 C2;
   typedef typename Mv<R>::V4 V4;
-  constexpr int NKS = 4 * SM, NH = NKS / 2, ST = SM * TM, NA = TM * NKS * 64;
-  __shared__ R s_A[FB][NA];
+  constexpr int NKS = 4 * SM, NH = NKS / 2, ST = SM * TM;
+  // LDS: [buffer][direction of the round][fb][plane][PL]; a plane's padding
+  // puts the planes that the rows of one tile read into different banks
+  constexpr int NV = 27 * ST, PL = NV + (NV % 4 == 2 ? 0 : (6 - NV % 4) % 4);
+  constexpr int NB = DS == 1 ? 2 : 1, SLOT = FB * 3 * PL;
+  constexpr int RED = DS == 1 ? 0 : (DS - 1) * FB * TM * 4 * 64;
+  __shared__ R s_T[NB * DS * SLOT > RED ? NB * DS * SLOT : RED];
+  constexpr int NT = M2LV_BS / DS, NI = (NV * FB + NT - 1) / NT;  // threads and values per thread of a staging
   // items (group of 8 frequencies, column block, FB-frequency run in the
-  // group): the runs of one 128-byte line of spectra run side by side on one XCD
+  // group): the runs of one group run side by side on one XCD
   constexpr int RUNS = 8 / FB;
   const int ngrp = (C + 7) / 8, nitem = ngrp * ncb * RUNS;
   const int item = xcd_item(blockIdx.x, nitem);
@@ -4061,96 +4084,131 @@ __global__ __launch_bounds__(M2LV_BS) void k_m2l_vec(int C, int Rc, long ncol, i
   if (item >= nitem || f0 >= C) return;  // block-uniform
   const int nf = min(FB, C - f0);
   const int t = threadIdx.x, w = t >> 6, l = t & 63, li = l & 15, lk = l >> 4;
-  const long col = ((long)cb * 4 + w) * 16 + li;
+  const int dw = DS == 1 ? 0 : w;  // the wave's direction slot of a round
+  const long col = ((long)cb * (4 / DS) + (DS == 1 ? w : 0)) * 16 + li;
   const int q = col < ncol ? (int)(col / Rc) : -1;
   const int r = col < ncol ? (int)(col - (long)(col / Rc) * Rc) : 0;
   const int msk = q >= 0 ? pmask[q] : 0;
   const int* ss = sslot + (long)(q < 0 ? 0 : q) * 26 * 8;
+  // the lane's A operand in a plane set: rbase (c, t, plane) + kofs (s, j)
+  int rb0[TM], rb1[TM], kofs[NH];
+#pragma unroll
+  for (int rt = 0; rt < TM; rt++) {
+    const int qo = rt * 8 + Mv<R>::row_out(li), c = qo / TM, ti = qo - c * TM, im = Mv<R>::row_im(li);
+    const int lc = (1 - (c >> 2)) * 9 + (1 - ((c >> 1) & 1)) * 3 + 1 - (c & 1);
+    rb0[rt] = dw * SLOT + lc * ST + ti * SM + (im ? 1 : 0) * PL;  // Yr = Mr Xr - Mi Xi, Yi = Mi Xr + Mr Xi
+    rb1[rt] = dw * SLOT + lc * ST + ti * SM + (im ? 0 : 2) * PL;
+  }
+#pragma unroll
+  for (int kh = 0; kh < NH; kh++) {
+    const int cs = kh * 4 + lk, s = cs / SM, j = cs - s * SM;
+    kofs[kh] = ((s >> 2) * 9 + ((s >> 1) & 1) * 3 + (s & 1)) * ST + j;
+  }
   V4 acc[FB][TM];
 #pragma unroll
   for (int fb = 0; fb < FB; fb++)
 #pragma unroll
     for (int rt = 0; rt < TM; rt++) acc[fb][rt] = V4{0, 0, 0, 0};
-  // operator-table entries and source slots of the next direction, loaded one
-  // direction ahead; the operator values and the source spectra of a
-  // direction are then fetched together, before its barriers
-  int ai[ST], sl[NH];
-  auto fetch_idx = [&](int n) {
-    if constexpr (!XA)
+  // direction n = (dx, dy, dz) - (1, 1, 1) in base 3, the centre left out
+  auto dir = [](int n, int& dx, int& dy, int& dz) {
+    const int m = n + (n >= 13);
+    dx = m / 9 - 1;
+    dy = m / 3 % 3 - 1;
+    dz = m % 3 - 1;
+  };
+  C2 tv[NI];
+  auto load_ops = [&](int n) {
+    int dx, dy, dz;
+    dir(n, dx, dy, dz);
+    const C2* base = opsT + ((long)f0 * 343 + (2 * dx + 2) * 49 + (2 * dy + 2) * 7 + 2 * dz + 2) * ST;
 #pragma unroll
-      for (int i = 0; i < ST; i++) ai[i] = aidx[(long)n * NA + t + M2LV_BS * i];
+    for (int i = 0; i < NI; i++) {
+      const int e = t % NT + NT * i, fb = e / NV, v = e - fb * NV, d = v / ST;
+      const int ex = d / 9, ey = d / 3 % 3, ez = d % 3;  // s - c + 1
+      // adjacent children: |2 n + s - c| <= 1 in every dimension
+      const bool adj = (dx == 0 || ex - 1 == -dx) && (dy == 0 || ey - 1 == -dy) && (dz == 0 || ez - 1 == -dz);
+      C2 x;
+      x.x = x.y = 0;
+      if (fb < nf && !adj) x = base[(long)fb * 343 * ST + (ex * 49 + ey * 7 + ez) * ST + v - d * ST];
+      tv[i] = x;
+    }
+  };
+  auto store_ops = [&](int buf) {
+    R* p = s_T + (buf * DS + (DS == 1 ? 0 : t / NT)) * SLOT;
+#pragma unroll
+    for (int i = 0; i < NI; i++) {
+      const int e = t % NT + NT * i, fb = e / NV, v = e - fb * NV, d = v / ST, j = (v - d * ST) / TM;
+      if (fb >= FB) continue;
+      R* o = p + fb * 3 * PL + d * ST + (v - d * ST - j * TM) * SM + j;
+      o[0] = tv[i].x;
+      o[PL] = tv[i].y;
+      o[2 * PL] = -tv[i].y;
+    }
+  };
+  int sl[NH];  // source slots of the next direction
+  auto load_slots = [&](int n) {
 #pragma unroll
     for (int kh = 0; kh < NH; kh++) sl[kh] = q >= 0 ? ss[n * 8 + (kh * 4 + lk) / SM] : -1;
   };
-  fetch_idx(0);
-  // the operators of the block's frequencies through a buffer resource based
-  // at frequency f0: one 32-bit byte offset per entry serves all FB
-  // frequencies, which lie a scalar FSTR bytes apart
-  constexpr unsigned FSTR = 343u * ST * sizeof(C2);
-  const __amdgpu_buffer_rsrc_t orsrc =
-      __builtin_amdgcn_make_buffer_rsrc((void*)(opsT + (long)f0 * 343 * ST), (short)0, (int)(FSTR * nf), BUF_DW3);
-  for (int n = 0; n < 26; n++) {
-    // the direction-n blocks [[Mr,-Mi],[Mi,Mr]] of the FB frequencies: entry
-    // e is aidx[n][e] = 2 x (index of the real value among one frequency's
-    // 343 sm tm complex operators) + 1 if negated, or -1 (adjacent pair)
-    R av[FB][ST];
-    if constexpr (XA) {
-#pragma unroll
-      for (int fb = 0; fb < FB; fb++) {
-        const R* ap = atabv + ((long)(f0 + (fb < nf ? fb : 0)) * 26 + n) * NA + t;
-#pragma unroll
-        for (int i = 0; i < ST; i++) av[fb][i] = ap[M2LV_BS * i];
-      }
-    } else {
-      unsigned ao[ST];
-#pragma unroll
-      for (int i = 0; i < ST; i++) ao[i] = (unsigned)(ai[i] < 0 ? 0 : ai[i] >> 1) * (unsigned)sizeof(R);
-#pragma unroll
-      for (int fb = 0; fb < FB; fb++)
-#pragma unroll
-        for (int i = 0; i < ST; i++) av[fb][i] = buf_ld<R>(orsrc, ao[i], fb < nf ? fb * (int)FSTR : 0);
-    }
-    // this lane's NH source spectra for the FB frequencies (contiguous in the
-    // spectra layout), clamped to slot 0 / the run and zeroed below
-    const bool use = __any((msk >> n) & 1);  // wave-uniform: a parent of the tile has direction n
+  constexpr int ROUNDS = (26 + DS - 1) / DS;
+  load_ops(dw);
+  load_slots(dw);
+  for (int i = 0; i < ROUNDS; i++) {
+    const int n = i * DS + dw, buf = NB == 2 ? i & 1 : 0;
+    const bool use = n < 26 && __any((msk >> (n < 26 ? n : 0)) & 1);  // wave-uniform
+    if (NB == 1 && i > 0) __syncthreads();  // the previous round is done with s_T
+    store_ops(buf);
     C2 x[NH][FB];
-    bool xz[NH];
+    bool have[NH];
     if (use) {
 #pragma unroll
       for (int kh = 0; kh < NH; kh++) {
-        const int j = (kh * 4 + lk) % SM;
-        xz[kh] = sl[kh] < 0;
-        const C2* xp = effden + (((long)(xz[kh] ? 0 : sl[kh]) * Rc + r) * SM + j) * C + f0;
+        have[kh] = sl[kh] >= 0;
+        const C2* xp = effden + ((((long)(have[kh] ? sl[kh] : 0) * Rc + r) * C + f0) * SM + (kh * 4 + lk) % SM);
 #pragma unroll
-        for (int fb = 0; fb < FB; fb++) x[kh][fb] = xp[fb < nf ? fb : 0];
+        for (int fb = 0; fb < FB; fb++) x[kh][fb] = xp[(fb < nf ? fb : 0) * SM];
       }
     }
-    // the entries' signs (waits for the operator values only: the spectra
-    // loads stay in flight), then the next direction's indices
-    if constexpr (!XA)
+    if (n + DS < 26) {
+      load_ops(n + DS);
+      load_slots(n + DS);
+    }
+    __syncthreads();
+    if (!use) continue;
+    const R* pT = s_T + buf * SLOT * DS;
+#pragma unroll
+    for (int kh = 0; kh < NH; kh++) {
+      if (!__any(have[kh])) continue;
+#pragma unroll
+      for (int fb = 0; fb < FB; fb++) {
+        const R xr = have[kh] ? x[kh][fb].x : (R)0, xi = have[kh] ? x[kh][fb].y : (R)0;
+#pragma unroll
+        for (int rt = 0; rt < TM; rt++) {
+          acc[fb][rt] = Mv<R>::mfma(pT[rb0[rt] + kofs[kh] + fb * 3 * PL], xr, acc[fb][rt]);
+          acc[fb][rt] = Mv<R>::mfma(pT[rb1[rt] + kofs[kh] + fb * 3 * PL], xi, acc[fb][rt]);
+        }
+      }
+    }
+  }
+  if constexpr (DS > 1) {  // partial sums of waves 1 .. DS - 1 into wave 0
+    __syncthreads();
+    if (w > 0)
 #pragma unroll
       for (int fb = 0; fb < FB; fb++)
 #pragma unroll
-        for (int i = 0; i < ST; i++) av[fb][i] = ai[i] < 0 ? (R)0 : ((ai[i] & 1) ? -av[fb][i] : av[fb][i]);
-    if (n + 1 < 26) fetch_idx(n + 1);
-    __syncthreads();  // the previous direction is done with s_A
+        for (int rt = 0; rt < TM; rt++)
 #pragma unroll
-    for (int fb = 0; fb < FB; fb++)
-#pragma unroll
-      for (int i = 0; i < ST; i++) s_A[fb][t + M2LV_BS * i] = av[fb][i];
+          for (int v = 0; v < 4; v++) s_T[((((w - 1) * FB + fb) * TM + rt) * 4 + v) * 64 + l] = acc[fb][rt][v];
     __syncthreads();
-    if (!use) continue;
+    if (w > 0) return;
 #pragma unroll
-    for (int kh = 0; kh < NH; kh++)
+    for (int o = 0; o < DS - 1; o++)
 #pragma unroll
-      for (int fb = 0; fb < FB; fb++) {
-        const R xr = xz[kh] ? (R)0 : x[kh][fb].x, xi = xz[kh] ? (R)0 : x[kh][fb].y;
+      for (int fb = 0; fb < FB; fb++)
 #pragma unroll
-        for (int rt = 0; rt < TM; rt++) {
-          acc[fb][rt] = Mv<R>::mfma(s_A[fb][(rt * NKS + kh) * 64 + l], xr, acc[fb][rt]);
-          acc[fb][rt] = Mv<R>::mfma(s_A[fb][(rt * NKS + kh + NH) * 64 + l], xi, acc[fb][rt]);
-        }
-      }
+        for (int rt = 0; rt < TM; rt++)
+#pragma unroll
+          for (int v = 0; v < 4; v++) acc[fb][rt][v] += s_T[(((o * FB + fb) * TM + rt) * 4 + v) * 64 + l];
   }
   if (q < 0) return;
 #pragma unroll
@@ -4160,88 +4218,67 @@ __global__ __launch_bounds__(M2LV_BS) void k_m2l_vec(int C, int Rc, long ncol, i
       const int qo = rt * 8 + Mv<R>::item_out(lk, h), c = qo / TM, ti = qo - c * TM;
       const int tl = tslot[(long)q * 8 + c];
       if (tl < 0) continue;
-      C2* out = effval + (((long)tl * Rc + r) * TM + ti) * C + f0;
+      C2* out = effval + (((long)tl * Rc + r) * C + f0) * TM + ti;
 #pragma unroll
       for (int fb = 0; fb < FB; fb++)
         if (fb < nf) {
           C2 v;
           v.x = acc[fb][rt][Mv<R>::item_re(h)];
           v.y = acc[fb][rt][Mv<R>::item_im(h)];
-          out[fb] = v;
+          out[fb * TM] = v;
         }
     }
 }
 
-template <class R, int SM, int TM, int FB>
+template <class R, int SM, int TM, int FB, int DS>
 static void m2l_vec_launch(hipStream_t s, int C, int npar, int Rc, const int* tslot, const int* sslot,
-                           const int* pmask, const int* aidx, const void* opsT, const void* atabv, const void* effden,
-                           void* effval)
+                           const int* pmask, const void* opsT, const void* effden, void* effval)
 {
   typedef typename Mv<R>::C2 C2;
-  const long ncol = (long)npar * Rc;
-  const int ncb = (int)((ncol + 63) / 64);
-  const dim3 grid(xcd_grid((C + 7) / 8 * ncb * (8 / FB)));
-  if constexpr (sizeof(R) == 4)
-    if (atabv) {
-      hipLaunchKernelGGL((k_m2l_vec<R, SM, TM, FB, true>), grid, dim3(M2LV_BS), 0, s, C, Rc, ncol, ncb, tslot, sslot,
-                         pmask, aidx, (const C2*)opsT, (const R*)atabv, (const C2*)effden, (C2*)effval);
-      return;
-    }
-  hipLaunchKernelGGL((k_m2l_vec<R, SM, TM, FB, false>), grid, dim3(M2LV_BS), 0, s, C, Rc, ncol, ncb, tslot, sslot,
-                     pmask, aidx, (const C2*)opsT, (const R*)nullptr, (const C2*)effden, (C2*)effval);
-}
-
-// atabv[(f * 26 + n) * na + e]: entry e of aidx[n] resolved against the
-// operators of frequency f (FP32, signs applied, zeros for -1)
-__global__ void k_expand_m2l_vec(int C, int na, int st, const int* __restrict__ aidx, const float* __restrict__ opsT,
-                                 float* __restrict__ atabv)
-{
-  const long n = (long)C * 26 * na;
-  for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
-    const long fn = i / na;
-    const int e = (int)(i - fn * na), f = (int)(fn / 26), d = (int)(fn - (long)f * 26);
-    const int ai = aidx[(long)d * na + e];
-    float v = 0.0f;
-    if (ai >= 0) {
-      v = opsT[(long)f * 343 * st * 2 + (ai >> 1)];
-      if (ai & 1) v = -v;
-    }
-    atabv[i] = v;
-  }
-}
-
-void expand_m2l_vec(hipStream_t s, int C, int sm, int tm, const int* aidx32, const float* opsT32, float* atabv)
-{
-  const int na = tm * 4 * sm * 64;
-  const long n = (long)C * 26 * na;
-  if (n <= 0) return;
-  hipLaunchKernelGGL(k_expand_m2l_vec, dim3(grid_for(n, 256)), dim3(256), 0, s, C, na, sm * tm, aidx32, opsT32, atabv);
+  const long ncol = (long)npar * Rc, per = 64 / DS;
+  const int ncb = (int)((ncol + per - 1) / per);
+  hipLaunchKernelGGL((k_m2l_vec<R, SM, TM, FB, DS>), dim3(xcd_grid((C + 7) / 8 * ncb * (8 / FB))), dim3(M2LV_BS), 0, s,
+                     C, Rc, ncol, ncb, tslot, sslot, pmask, (const C2*)opsT, (const C2*)effden, (C2*)effval);
 }
 
 template <class R>
 static void m2l_matrix_t(hipStream_t s, int sm, int tm, int C, int npar, int Rc, const int* tslot, const int* sslot,
-                         const int* pmask, const int* aidx, const void* opsT, const void* atabv, const void* effden,
-                         void* effval)
+                         const int* pmask, const void* opsT, const void* effden, void* effval)
 {
-  // frequencies per block: 2 measured best in both precisions (of 1, 2, 4, 8)
-  constexpr int FB = 2;
-  if (sm == 1 && tm == 1)
-    m2l_vec_launch<R, 1, 1, FB>(s, C, npar, Rc, tslot, sslot, pmask, aidx, opsT, atabv, effden, effval);
-  else if (sm == 4 && tm == 3)
-    m2l_vec_launch<R, 4, 3, FB>(s, C, npar, Rc, tslot, sslot, pmask, aidx, opsT, atabv, effden, effval);
-  else if (sm == 3 && tm == 3)
-    m2l_vec_launch<R, 3, 3, FB>(s, C, npar, Rc, tslot, sslot, pmask, aidx, opsT, atabv, effden, effval);
+  // Frequencies per block: FP32 vector kernels 2 (1: Navier clusters 28.8 ->
+  // 32.1 ms a pass, 4: the same), FP64 ones 1 (128 VGPRs instead of 218: Stokes
+  // sphere 8.21 -> 7.96 ms a pass, 4: 8.90), scalar kernels 4.  Scalar FP64
+  // levels of fewer than 1024 blocks split the directions over the waves, 2
+  // frequencies per block (3k / 65k Laplace a pass: 526 / 847 us unsplit, 497 /
+  // 797 with 4 frequencies, 473 / 780 with 2; split, the vector kernels were
+  // slower).  The FP32 sums keep one chain over the directions.
+  constexpr bool F64 = sizeof(R) == 8;
+#define KIFMM_M2LV(SM, TM, FB, DS) \
+  m2l_vec_launch<R, SM, TM, FB, DS>(s, C, npar, Rc, tslot, sslot, pmask, opsT, effden, effval)
+  if (sm == 1 && tm == 1) {
+    const long nblock = ((long)npar * Rc + 63) / 64 * ((C + 3) / 4);
+    if constexpr (F64)
+      if (nblock < 1024) {
+        KIFMM_M2LV(1, 1, 2, 4);
+        return;
+      }
+    KIFMM_M2LV(1, 1, 4, 1);
+  } else if (sm == 4 && tm == 3) {
+    KIFMM_M2LV(4, 3, (F64 ? 1 : 2), 1);
+  } else if (sm == 3 && tm == 3) {
+    KIFMM_M2LV(3, 3, (F64 ? 1 : 2), 1);
+  }
+#undef KIFMM_M2LV
 }
 
 void m2l_matrix(hipStream_t s, int sm, int tm, int C, int npar, int Rc, const int* tslot, const int* sslot,
-                const int* pmask, const int* aidx, const void* opsT, const void* atabv, const void* effden,
-                void* effval, int single)
+                const int* pmask, const void* opsT, const void* effden, void* effval, int single)
 {
   if (npar <= 0) return;
   if (single)
-    m2l_matrix_t<float>(s, sm, tm, C, npar, Rc, tslot, sslot, pmask, aidx, opsT, atabv, effden, effval);
+    m2l_matrix_t<float>(s, sm, tm, C, npar, Rc, tslot, sslot, pmask, opsT, effden, effval);
   else
-    m2l_matrix_t<double>(s, sm, tm, C, npar, Rc, tslot, sslot, pmask, aidx, opsT, nullptr, effden, effval);
+    m2l_matrix_t<double>(s, sm, tm, C, npar, Rc, tslot, sslot, pmask, opsT, effden, effval);
 }
 
 }  // namespace dev

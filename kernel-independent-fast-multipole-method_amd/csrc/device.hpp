@@ -151,11 +151,13 @@ double cmp_sigma(double abs_row_sum);
 int gemm_split(const GemmArgs& a);
 
 // r2c of the scaled upward equivalent densities on the (2np)^3 grid into
-// complex spectra, effden[slot][Rc][sm][C] (rhs_inner 0) or
-// effden[slot][sm][C][Rc] (rhs_inner 1), stored as double2 or, with single,
-// as float2.
+// complex spectra, stored as double2 or, with single, as float2, in the layout
+// that the level's M2L form reads:
+constexpr int SPEC_FREQ_INNER = 0;  // [slot][Rc][sm][C]: grouped and per-pair VALU forms
+constexpr int SPEC_RHS_INNER = 1;   // [slot][sm][C][Rc]: tiled and wave matrix-core forms
+constexpr int SPEC_DOF_INNER = 2;   // [slot][Rc][C][sm]: parent-grouped matrix-core form
 void fft_fwd(hipStream_t s, int np, int nslot, const int* slot_node, int Rc, const double* upeden, int pln, int sm,
-             const double* dscale, const short* cube2surf, void* effden, int single, int rhs_inner,
+             const double* dscale, const short* cube2surf, void* effden, int single, int layout,
              const double2* tw);
 // M2L products summed over V pairs -> effval[trg][Rc][tm][C] (overwritten).
 void m2l(hipStream_t s, int sm, int tm, int C, int ntrg, int Rc, const int* vptr, const int* vsrc, const int* vop,
@@ -167,25 +169,18 @@ void m2l(hipStream_t s, int sm, int tm, int C, int ntrg, int Rc, const int* vptr
 void m2l_grouped(hipStream_t s, int sm, int tm, int C, int npar, int Rc, int rb, int bs, const int* tslot,
                  const int* sslot, const int* optab, const double2* ops, const double2* effden, double2* effval);
 // The same sums on the matrix cores: columns (parent, right-hand side) in
-// tiles of 16, operators from the frequency-major copy opsT [C][343][sm][tm];
-// pmask[p] bit n set if parent p has a source child in direction n; aidx
-// [26][tm][4 sm][64] the A-operand table of the precision's row layout
-// (2 x index of the real value among one frequency's operators + 1 if
-// negated, -1 for zero).  single selects FP32 spectra and operators (float2,
-// all directions accumulated in FP32), otherwise FP64 (double2).  atabv: the
-// FP32 A operands expanded by expand_m2l_vec, used by the FP32 form when not
-// null (the FP64 form resolves aidx against opsT).
+// tiles of 16, spectra [slot][Rc][C][sm] and [slot][Rc][C][tm], operators from
+// the frequency-major copy opsT [C][343][sm][tm]; pmask[p] bit n set if parent
+// p has a source child in direction n.  single selects FP32 spectra and
+// operators (float2, all directions accumulated in FP32), otherwise FP64
+// (double2).
 void m2l_matrix(hipStream_t s, int sm, int tm, int C, int npar, int Rc, const int* tslot, const int* sslot,
-                const int* pmask, const int* aidx, const void* opsT, const void* atabv, const void* effden,
-                void* effval, int single);
-// atabv [C][26][tm 4 sm 64] = the FP32 A-operand table aidx32 resolved
-// against the FP32 operators opsT32 of every frequency
-void expand_m2l_vec(hipStream_t s, int C, int sm, int tm, const int* aidx32, const float* opsT32, float* atabv);
+                const int* pmask, const void* opsT, const void* effden, void* effval, int single);
 // c2r and gather onto the DC surface: dncval[(node*Rc + r)*pln + p*tm + f] = ...
 // (assigned: every DC value of the listed nodes; effval in the layout and
 // precision described for fft_fwd)
 void fft_inv(hipStream_t s, int np, int nslot, const int* slot_node, int Rc, const void* effval, int single,
-             int rhs_inner, int tm, const int* surf2cube, int nsp, double* dncval, int pln, const double2* tw);
+             int layout, int tm, const int* surf2cube, int nsp, double* dncval, int pln, const double2* tw);
 // Tiled M2L on the matrix cores for scalar kernels, spectra with the
 // right-hand sides innermost and Rc a multiple of 16: for every tile (2x2x2
 // target parents, ttile [ntile][8][8] child slots) and its 4x4x4 halo of

@@ -352,11 +352,6 @@ void Engine::upload_static()
   tw_.upload(tw);
   I_.upload(plan_.I);
   D_.upload(plan_.D);
-  {  // FP32 A operands of the parent-grouped M2L, expanded per (frequency, direction)
-    const size_t na = (size_t)mm_.tdof * 4 * mm_.sdof * 64;
-    avec32_.alloc((size_t)O.C * 26 * na);
-    dev::expand_m2l_vec(stream_, O.C, mm_.sdof, mm_.tdof, I_.p + plan_.aidx[1], opsT32_.p, avec32_.p);
-  }
   {  // fused operator of the mixed up pass: m2me_ = UC2UE x [UE2UC_0 .. UE2UC_7],
      // compensated like the pseudoinverse applies
     const int pUE = O.pln[SURF_UE], pUC = O.pln[SURF_UC];
@@ -676,31 +671,6 @@ void Engine::build_plan()
             }
     }
     P.optab = pool_i(P.I, optab);
-    // A-operand tables of the parent-grouped matrix-core M2L: entry (n, rt,
-    // ks, lane) of the real embedding [[Mr, -Mi], [Mi, Mr]] of the direction-n
-    // operator block, for the FP64 row layout (row r16 = output r16 % 8, part
-    // r16 / 8) and the FP32 one (output r16 / 2, part r16 % 2)
-    for (int prec = 0; prec < 2; prec++) {
-      const int tmv = mm_.tdof, nks = 4 * sm;
-      std::vector<int> aidx((size_t)26 * tmv * nks * 64, -1);
-      for (int n = 0; n < 26; n++)
-        for (int rt = 0; rt < tmv; rt++)
-          for (int ks = 0; ks < nks; ks++)
-            for (int ll = 0; ll < 64; ll++) {
-              const int r16 = ll & 15, kk = ll >> 4;
-              const int ro = prec == 0 ? (r16 & 7) : (r16 >> 1);
-              const bool imrow = prec == 0 ? r16 >= 8 : (r16 & 1) == 1;
-              const int qo = rt * 8 + ro, c = qo / tmv, ti = qo % tmv;
-              const int kap = ks * 4 + kk, pin = kap / (8 * sm), cs = kap % (8 * sm), sc = cs / sm, j = cs % sm;
-              const int o = optab[(n * 8 + sc) * 8 + c];
-              if (o < 0) continue;
-              const int part = imrow ? (pin == 0 ? 1 : 0) : pin;  // Yr = Mr Xr - Mi Xi, Yi = Mi Xr + Mr Xi
-              const int neg = (!imrow && pin == 1) ? 1 : 0;
-              const int vidx = ((o * sm + j) * tmv + ti) * 2 + part;
-              aidx[(((size_t)n * tmv + rt) * nks + ks) * 64 + ll] = vidx * 2 + neg;
-            }
-      P.aidx[prec] = pool_i(P.I, aidx);
-    }
     std::vector<int> sslot_of(T.nnode, -1), tslot_of(T.nnode, -1);
     for (int L = 2; L < T.nlevel; L++) {
       std::vector<int> trg, src, vptr(1, 0), vsrc, vop;
@@ -1517,11 +1487,12 @@ void Engine::run_chunk(const double* srcden, double* trgval, int rc, int mode, h
     const VLevel& vl = P.vlev[li];
     const int form = m2l_form(mixed, li, rc);
     const bool tiled = form == 0 || form == 4;
-    const int ri = tiled ? 1 : 0, single = mixed && (form <= 1 || form == 4) ? 1 : 0;
+    const int layout = tiled ? dev::SPEC_RHS_INNER : form == 1 ? dev::SPEC_DOF_INNER : dev::SPEC_FREQ_INNER;
+    const int single = mixed && (form <= 1 || form == 4) ? 1 : 0;
     cur_lvl = (int)li;
     timed(KIFMM3D_K_FFT_FWD, [&] {
       dev::fft_fwd(s, np_, vl.nsrc, I + vl.src_node, rc, upeden_.p, pUE, sm, D + vl.dscale, c2s_.p, effden_.p, single,
-                   ri, (const double2*)tw_.p);
+                   layout, (const double2*)tw_.p);
     });
     timed(KIFMM3D_K_M2L, [&] {
       if (form == 4) {
@@ -1540,15 +1511,14 @@ void Engine::run_chunk(const double* srcden, double* trgval, int rc, int mode, h
         dev::m2l(s, sm, tm, O.C, vl.ntrg, rc, I + vl.vptr, I + vl.vsrc, I + vl.vop, (const double2*)m2l_.p,
                  (const double2*)effden_.p, (double2*)effval_.p);
       else if (form == 1)
-        dev::m2l_matrix(s, sm, tm, O.C, vl.npar, rc, I + vl.tslot, I + vl.sslot, I + vl.pmask, I + P.aidx[single],
-                        single ? (const void*)opsT32_.p : (const void*)opsT_.p, avec32_.p, effden_.p, effval_.p,
-                        single);
+        dev::m2l_matrix(s, sm, tm, O.C, vl.npar, rc, I + vl.tslot, I + vl.sslot, I + vl.pmask,
+                        single ? (const void*)opsT32_.p : (const void*)opsT_.p, effden_.p, effval_.p, single);
       else
         dev::m2l_grouped(s, sm, tm, O.C, vl.npar, rc, m2l_rb_, m2l_bs_, I + vl.tslot, I + vl.sslot, I + P.optab,
                          (const double2*)m2l_.p, (const double2*)effden_.p, (double2*)effval_.p);
     });
     timed(KIFMM3D_K_FFT_INV, [&] {
-      dev::fft_inv(s, np_, vl.ntrg, I + vl.trg_node, rc, effval_.p, single, ri, tm, s2c_.p, O.nsp[SURF_DC],
+      dev::fft_inv(s, np_, vl.ntrg, I + vl.trg_node, rc, effval_.p, single, layout, tm, s2c_.p, O.nsp[SURF_DC],
                    dncval_.p, pDC, (const double2*)tw_.p);
     });
     cur_lvl = -1;

@@ -100,7 +100,6 @@ struct Plan {
   int max_vsrc = 0, max_vtrg = 0;
   bool m2l_pairs = false;      // per-pair M2L kernel instead of the parent-grouped one
   size_t optab = 0;            // [26 directions][8 source children][8 target children] -> operator or -1
-  size_t aidx[2] = {0, 0};     // A-operand tables of the matrix-core M2L, FP64 and FP32 row layouts
   int nlow_s = 0, nlow_t = 0;  // source / target node indices of depth < 2 form these prefixes
   long near_pairs = 0;         // source-target pairs of the near field (one RHS)
   long far_pairs = 0;          // surface point - target pairs of L2T + M2T
@@ -267,7 +266,6 @@ class Engine {
   DVec<double> atab_;  // tiled M2L A-operand tables [C][26 x 32][2] complex (scalar kernels)
   DVec<float> atab32_;  // the same in FP32
   DVec<float> opsT32_; // the same in FP32
-  DVec<float> avec32_; // FP32 A operands of the parent-grouped M2L, [C][26][tdof 4 sdof 64]
   DVec<double> tw_;
   DVec<int> I_;
   DVec<double> D_;
