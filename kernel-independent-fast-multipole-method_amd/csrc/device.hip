@@ -2569,6 +2569,124 @@ constexpr int GMX_RT = 10, GMX_G = 2;
 
 // Splits of K that bring a wide-tile product to about a.split_blocks blocks
 // (default 1024, 4 per CU; 1 = no split; each split keeps at least 4 steps of 8).
+// The same product for few columns: a block forms 32 x 32 of C with one wave per
+// split of K (ks of them, k_gemm_mx's splits in its order of operations, so the
+// two agree to the bit), each wave's A and B operands straight from global
+// memory, two steps of 8 ahead; the waves' sums are added in LDS in split order.
+// Where the columns fill the chip only by splitting K the wide tile is bound by
+// latency, not by rate: mostly padding (1 to 60 columns of 128) on the upper
+// levels, one wave per SIMD whose every step waits for a staged load, and a
+// second launch and a round trip through memory for the partial sums.  All
+// products of a pass: 262k Stokes sphere (mixed) 1.90 -> 1.16 ms, 1M Navier
+// clusters 8.5 -> 6.3 ms, clusters at 21 right-hand sides up + down 5.6 -> 4.8.
+// M <= 64 (np 4), whose wide tile is 256 columns: the same up to 512 tiles (65k
+// mixed, a pass: 485 -> 417 us), slower above (65k plain 703 -> 721 us).
+template <int KS>
+__global__ __launch_bounds__(64 * KS) void k_gemm_sm(GemmArgs p, int ks)
+{
+  constexpr int LD = 33;  // padded column of the LDS sums
+  __shared__ double s_sum[KS * 32 * LD];
+  const int grp = blockIdx.z;
+  const int n0 = p.gbeg[grp], n1 = p.gbeg[grp + 1];
+  const long cb = (long)n0 * p.Rc + (long)blockIdx.x * 32, ce = (long)n1 * p.Rc;
+  if (cb >= ce) return;  // block-uniform
+  const int rb = blockIdx.y * 32;
+  const int t = threadIdx.x, w = t >> 6, l = t & 63, li = l & 15, lk = l >> 4;
+  const int nstep = p.nseg * p.Kseg / 8, sps = p.Kseg / 8;
+  const int st0 = (int)((long)nstep * w / ks), st1 = (int)((long)nstep * (w + 1) / ks);
+  // rows and columns past the end: the first ones, whose products are not stored
+  const double* ap[2];
+#pragma unroll
+  for (int rt = 0; rt < 2; rt++) {
+    const int row = rb + rt * 16 + li;
+    ap[rt] = p.A + grp * p.a_gstride + (row < p.M ? row : 0);
+  }
+  int cn[2], cr[2];
+  bool cok[2];
+#pragma unroll
+  for (int g = 0; g < 2; g++) {
+    const long j = cb + g * 16 + li;
+    cok[g] = j < ce;
+    cn[g] = cok[g] ? (int)(j / p.Rc) : 0;
+    cr[g] = cok[g] ? (int)(j - (long)cn[g] * p.Rc) : 0;
+  }
+  const double* bp[2];
+  double bm[2];
+  auto seg_ptrs = [&](int seg) {
+    const double* Bb = (seg > 0 && p.B2) ? p.B2 : p.B;
+#pragma unroll
+    for (int g = 0; g < 2; g++) {
+      const int bn = cok[g] ? p.bnode[(long)seg * p.ncol + cn[g]] : -1;
+      bp[g] = Bb + (bn >= 0 ? ((long)bn * p.Rc + cr[g]) * p.Kseg : 0) + 2 * lk;
+      bm[g] = bn >= 0 ? 1.0 : 0.0;
+    }
+  };
+  struct Step {
+    double a[2][2];
+    double2 b[2];
+  };
+  auto load = [&](int st, Step& x) {
+    if (st == st0 || st % sps == 0) seg_ptrs(st / sps);
+    const int seg = st / sps, kin = (st - seg * sps) * 8;
+#pragma unroll
+    for (int sl = 0; sl < 2; sl++)
+#pragma unroll
+      for (int rt = 0; rt < 2; rt++) x.a[sl][rt] = ap[rt][(long)(st * 8 + 2 * lk + sl) * p.M];
+#pragma unroll
+    for (int g = 0; g < 2; g++) {
+      const double2 v = *(const double2*)(bp[g] + kin);
+      x.b[g] = make_double2(v.x * bm[g], v.y * bm[g]);
+    }
+    if (p.bscale && seg >= p.bscale_seg)  // powers of two: exact on either operand
+#pragma unroll
+      for (int sl = 0; sl < 2; sl++)
+#pragma unroll
+        for (int rt = 0; rt < 2; rt++) x.a[sl][rt] *= p.bscale[kin + 2 * lk + sl];
+  };
+  v4d acc[2][2];
+#pragma unroll
+  for (int rt = 0; rt < 2; rt++)
+#pragma unroll
+    for (int g = 0; g < 2; g++) acc[rt][g] = v4d{0.0, 0.0, 0.0, 0.0};
+  auto apply = [&](const Step& x) {
+#pragma unroll
+    for (int sl = 0; sl < 2; sl++)
+#pragma unroll
+      for (int rt = 0; rt < 2; rt++)
+#pragma unroll
+        for (int g = 0; g < 2; g++)
+          acc[rt][g] = __builtin_amdgcn_mfma_f64_16x16x4f64(x.a[sl][rt], sl ? x.b[g].y : x.b[g].x, acc[rt][g], 0, 0, 0);
+  };
+  Step x0, x1;
+  if (st0 < st1) load(st0, x0);
+  if (st0 + 1 < st1) load(st0 + 1, x1);
+  for (int st = st0; st < st1; st += 2) {  // wave-uniform
+    apply(x0);
+    if (st + 2 < st1) load(st + 2, x0);
+    if (st + 1 < st1) apply(x1);
+    if (st + 3 < st1) load(st + 3, x1);
+  }
+  double* d = s_sum + w * 32 * LD;
+#pragma unroll
+  for (int rt = 0; rt < 2; rt++)
+#pragma unroll
+    for (int g = 0; g < 2; g++)
+#pragma unroll
+      for (int v = 0; v < 4; v++) d[(g * 16 + li) * LD + rt * 16 + lk + 4 * v] = acc[rt][g][v];
+  __syncthreads();
+  for (int e = t; e < 1024; e += 64 * ks) {
+    const int c = e >> 5, row = rb + (e & 31);
+    const long jj = cb + c;
+    if (row >= p.M || jj >= ce) continue;
+    double h = 0.0;
+    for (int sp = 0; sp < ks; sp++) h += s_sum[sp * 32 * LD + c * LD + (e & 31)];
+    if (p.cscale) h *= p.cscale[row];  // power of two: exact
+    const long n = jj / p.Rc;
+    double* out = p.C + ((long)p.cnode[n] * p.Rc + (jj - n * p.Rc)) * p.M + row;
+    *out = p.accumulate ? *out + h : h;
+  }
+}
+
 static int gemm_split_of(const GemmArgs& a, long nb)
 {
   const long target = a.split_blocks > 0 ? a.split_blocks : 1024;
@@ -2601,6 +2719,17 @@ void gemm(hipStream_t s, const GemmArgs& a)
   // workspace
   if (a.mfma == 2 && a.Kseg % 8 == 0) {
     int ks = gemm_split(a);
+    const long n32 = (long)((a.M + 31) / 32) * ((cols + 31) / 32) * a.ngroup;
+    if (ks > 1 && (a.M > 64 || n32 <= 512)) {
+      const dim3 grid((unsigned)((cols + 31) / 32), (unsigned)((a.M + 31) / 32), (unsigned)a.ngroup), bs(64 * ks);
+      if (ks <= 4)
+        hipLaunchKernelGGL(k_gemm_sm<4>, grid, bs, 0, s, a, ks);
+      else if (ks <= 8)
+        hipLaunchKernelGGL(k_gemm_sm<8>, grid, bs, 0, s, a, ks);
+      else
+        hipLaunchKernelGGL(k_gemm_sm<16>, grid, bs, 0, s, a, ks);
+      return;
+    }
     if (a.B2 && !(a.work && (long)ks * a.ctot * a.M <= a.work_n)) ks = 1;  // two B buffers: wide tiles only
     if (ks == 1 || (a.work && (long)ks * a.ctot * a.M <= a.work_n)) {
       if (a.M <= 64) {
