@@ -1018,7 +1018,7 @@ void Engine::record(const double* d_srcden, double* d_trgval, int nrhs, int rc, 
   if (nt_ == 0) return;
   for (int r0 = 0; r0 < nrhs; r0 += rc) {
     const int n = std::min(rc, nrhs - r0);
-    run_chunk(d_srcden + (size_t)r0 * ns_ * user_.sdof, d_trgval + (size_t)r0 * nt_ * user_.tdof, n, mode, s, nullptr);
+    run_chunk(d_srcden + (size_t)r0 * ns_ * user_.sdof, d_trgval + (size_t)r0 * nt_ * user_.tdof, n, mode, s, false);
     last_rc_ = n;
   }
 }
@@ -1078,33 +1078,25 @@ void Engine::evaluate_device(const double* d_srcden, double* d_trgval, int nrhs,
     return;
   }
   vlev_ms_.assign(plan_.vlev.size(), 0.0);
-  hipEvent_t ev[9];
-  for (auto& e : ev) HIPCHK(hipEventCreate(&e));
-  try {
-    for (int r0 = 0; r0 < nrhs; r0 += rc) {
-      int n = std::min(rc, nrhs - r0);
-      run_chunk(d_srcden + (size_t)r0 * ns_ * user_.sdof, d_trgval + (size_t)r0 * nt_ * user_.tdof, n, mode, stream_,
-                ev);
-      HIPCHK(hipEventSynchronize(ev[8]));
-      for (int s = 0; s < 8; s++) {
-        float ms = 0;
-        HIPCHK(hipEventElapsedTime(&ms, ev[s], ev[s + 1]));
-        stage_ms[s] += ms;
-      }
-      for (size_t e = 0; e + 1 < nev_used_; e += 2) {
-        float ms = 0;
-        HIPCHK(hipEventElapsedTime(&ms, evpool_[e], evpool_[e + 1]));
-        kernel_ms[evcls_[e / 2]] += ms;
-        kernel_calls[evcls_[e / 2]] += 1;
-        if (evlvl_[e / 2] >= 0) vlev_ms_[evlvl_[e / 2]] += ms;
-      }
-      last_rc_ = n;
+  for (int r0 = 0; r0 < nrhs; r0 += rc) {
+    int n = std::min(rc, nrhs - r0);
+    run_chunk(d_srcden + (size_t)r0 * ns_ * user_.sdof, d_trgval + (size_t)r0 * nt_ * user_.tdof, n, mode, stream_,
+              true);
+    HIPCHK(hipEventSynchronize(evpool_[evmark_[8]]));
+    auto between = [&](int from, int to) {
+      float ms = 0;
+      if (from != to) HIPCHK(hipEventElapsedTime(&ms, evpool_[from], evpool_[to]));
+      return ms;
+    };
+    for (int s = 0; s < 8; s++) stage_ms[s] += between(evmark_[s], evmark_[s + 1]);
+    for (const TimedLaunch& l : evlog_) {
+      const float ms = between(l.from, l.to);
+      kernel_ms[l.cls] += ms;
+      kernel_calls[l.cls] += 1;
+      if (l.lvl >= 0) vlev_ms_[l.lvl] += ms;
     }
-  } catch (...) {
-    for (auto& e : ev) (void)hipEventDestroy(e);
-    throw;
+    last_rc_ = n;
   }
-  for (auto& e : ev) (void)hipEventDestroy(e);
   double tot = 0;
   for (int s = 0; s < 8; s++) tot += stage_ms[s];
   stage_ms[KIFMM3D_STAGE_TOTAL] = tot;
@@ -1355,7 +1347,7 @@ int Engine::settings(int mode, int* out, int n) const
   return cnt;
 }
 
-void Engine::run_chunk(const double* srcden, double* trgval, int rc, int mode, hipStream_t s, hipEvent_t* ev)
+void Engine::run_chunk(const double* srcden, double* trgval, int rc, int mode, hipStream_t s, bool time)
 {
   const bool mixed = mode == KIFMM3D_MODE_MIXED;
   const Operators& O = *ops_;
@@ -1406,33 +1398,42 @@ void Engine::run_chunk(const double* srcden, double* trgval, int rc, int mode, h
     dev::gemm(s, a);
   };
 
-  // stage and kernel-class timing: events on this stream (none when ev is
-  // null, e.g. while the sequence is captured into a graph)
-  auto mark = [&](int k) {
-    if (ev) HIPCHK(hipEventRecord(ev[k], s));
+  // Stage and kernel-class timing: events on this stream (none without time,
+  // e.g. while the sequence is captured into a graph).  An event between two
+  // launches holds the second back by several microseconds, so adjoining
+  // intervals share one: stamp() records only if something was enqueued since
+  // the last.  Only event 0, the last of an evaluate, carries the fence that
+  // makes the results visible outside the device.
+  int nev = 1, cur = -1;
+  bool fresh = false;  // nothing enqueued on s since event cur
+  auto new_event = [&](hipStream_t st) {
+    while ((int)evpool_.size() <= nev) {
+      hipEvent_t e;
+      HIPCHK(hipEventCreateWithFlags(&e, evpool_.empty() ? hipEventDefault : hipEventDisableSystemFence));
+      evpool_.push_back(e);
+    }
+    HIPCHK(hipEventRecord(evpool_[nev], st));
+    return nev++;
   };
-  size_t nev = 0;
+  auto stamp = [&] {
+    if (!fresh) cur = new_event(s);
+    fresh = true;
+    return cur;
+  };
+  auto mark = [&](int k) {
+    if (time) evmark_[k] = stamp();
+  };
+  evlog_.clear();
   int cur_lvl = -1;  // V-list level being enqueued (for the per-level times)
   auto timed_on = [&](hipStream_t st, int cls, auto&& fn) {
-    if (!ev) {
+    if (!time) {
       fn();
       return;
     }
-    if (evpool_.size() < nev + 2) {
-      hipEvent_t a, b;
-      HIPCHK(hipEventCreate(&a));
-      HIPCHK(hipEventCreate(&b));
-      evpool_.push_back(a);
-      evpool_.push_back(b);
-    }
-    HIPCHK(hipEventRecord(evpool_[nev], st));
+    const int from = st == s ? stamp() : new_event(st);
     fn();
-    HIPCHK(hipEventRecord(evpool_[nev + 1], st));
-    evcls_.resize(nev / 2 + 1);
-    evcls_[nev / 2] = cls;
-    evlvl_.resize(nev / 2 + 1);
-    evlvl_[nev / 2] = cur_lvl;
-    nev += 2;
+    if (st == s) fresh = false;
+    evlog_.push_back({from, st == s ? stamp() : new_event(st), cls, cur_lvl});
   };
   auto timed = [&](int cls, auto&& fn) { timed_on(s, cls, fn); };
 
@@ -1445,6 +1446,7 @@ void Engine::run_chunk(const double* srcden, double* trgval, int rc, int mode, h
   if (P.nlow_s) dev::zero(s, upcval_.p, (long)rc * P.nlow_s * pUC);
   if (P.nlow_s) dev::zero(s, upeden_.p, (long)rc * P.nlow_s * pUE);
   if (P.nlow_t) dev::zero(s, dneden_.p, (long)rc * P.nlow_t * pDE);
+  fresh = false;
   // load (fmm3d_eval.cpp:50-64)
   timed(KIFMM3D_K_GATHER,
         [&] { dev::gather(s, T.sextcnt, sdof, rc, siperm_.p, srcden, (long)ns_ * sdof, den64, den32); });
@@ -1535,7 +1537,10 @@ void Engine::run_chunk(const double* srcden, double* trgval, int rc, int mode, h
   for (const GemmOp& op : mixed && !P.down_mixed.empty() ? P.down_mixed : P.down)
     timed(KIFMM3D_K_GEMM_DOWN, [&] { run_gemm(op); });
   mark(6);
-  if (side) HIPCHK(hipStreamWaitEvent(s, join_ev_, 0));
+  if (side) {
+    HIPCHK(hipStreamWaitEvent(s, join_ev_, 0));
+    fresh = false;
+  }
   // L2T + M2T
   timed(KIFMM3D_K_S2P, [&] {
     const auto far = [&](const ChunkList& l) {
@@ -1553,8 +1558,10 @@ void Engine::run_chunk(const double* srcden, double* trgval, int rc, int mode, h
       dev::scatter(s, T.textcnt, tdof, rc, tperm_.p, tval_.p, trs, trgval, (long)nt_ * tdof);
   });
   HIPCHK(hipGetLastError());
-  mark(8);
-  if (ev) nev_used_ = nev;
+  if (time) {
+    evmark_[8] = 0;
+    HIPCHK(hipEventRecord(evpool_[0], s));
+  }
 }
 
 long Engine::get_buffer(int what, double* buf, long n)

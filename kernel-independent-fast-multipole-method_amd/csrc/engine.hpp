@@ -195,7 +195,7 @@ class Engine {
   // effval, gwork (doubles), sden32 (floats; 0 unless Laplace).
   static constexpr int NWORK = 11;
   void work_counts(int rc, size_t cnt[NWORK]) const;
-  void run_chunk(const double* srcden, double* trgval, int rc, int mode, hipStream_t s, hipEvent_t* ev);
+  void run_chunk(const double* srcden, double* trgval, int rc, int mode, hipStream_t s, bool time);
   void drop_graph();
   int near_variant(bool mixed) const;
   // The FP32 vector near field (kernel 4) is the mixed form's for the 1/r
@@ -241,13 +241,17 @@ class Engine {
   double* gtrg_ = nullptr;
   int gnrhs_ = 0, gmode_ = -1, grc_ = 0;
   unsigned long ggen_ = 0;
+  // events of the last timed chunk: those of the stage boundaries, and from
+  // and to of every timed launch with its class and V-list level (-1 outside)
+  struct TimedLaunch {
+    int from, to, cls, lvl;
+  };
   std::vector<hipEvent_t> evpool_;
-  std::vector<int> evcls_;
-  std::vector<int> evlvl_;        // V-list level of each timed launch (-1 outside the V list)
+  std::vector<TimedLaunch> evlog_;
+  int evmark_[9] = {0};
   std::vector<double> vlev_ms_;   // per V-list level: FFTs + M2L of the last timed evaluate
   int p2p_tuned_[2] = {-1, -1};   // per mode: tuned near-field kernel (-1: default)
   std::vector<int> m2l_form_[2];  // per mode, per V-list level: tuned M2L form (empty: default)
-  size_t nev_used_ = 0;
 
   // device data
   DVec<double> sx_, sy_, sz_, snx_, sny_, snz_, tx_, ty_, tz_;
