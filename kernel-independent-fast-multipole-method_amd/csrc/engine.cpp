@@ -104,7 +104,7 @@ Engine::Engine(int kt, const double* coefs, int ncoefs, int np, int ptsmax, int 
     const std::string v(m);
     m2l_tile_ = v != "group" && v != "pair" && v != "matrix";
     m2l_matrix_ = v != "group" && v != "pair";
-    m2l_wave_ = v == "wave";
+    m2l_wave_ = v == "wave" ? 1 : 0;
   }
   if (const char* d = std::getenv("KIFMM3D_M2L_DEPTH")) m2l_depth_ = std::atoi(d);
   if (const char* d = std::getenv("KIFMM3D_M2L_FPART")) m2l_fpart_ = std::atoi(d);
@@ -1233,7 +1233,13 @@ int Engine::m2l_form(bool mixed, size_t level, int rc) const
   const std::vector<int>& tf = m2l_form_[mixed ? 1 : 0];
   if (level < tf.size() && tf[level] >= 0 && ((tf[level] != 0 && tf[level] != 4) || tile_ok))
     return tf[level];
-  return m2l_tile_ && tile_ok ? (m2l_wave_ ? 4 : 0) : m2l_matrix_ ? 1 : 2;
+  // Untuned: the wave-per-tile form in FP64, on every level (16 right-hand
+  // sides, M2L of a pass, block per tile / wave per tile: 30k cube 0.20 / 0.08
+  // ms, 300k cube 2.68 / 1.58, 200k clusters 8.3 / 4.3, 200k sphere 5.8 / 3.4,
+  // 300k clusters at np 8 24.1 / 10.4); the mixed form keeps the block-per-tile
+  // one, whose FP32 sums run in another order.
+  const bool wave = m2l_wave_ < 0 ? !mixed : m2l_wave_ != 0;
+  return m2l_tile_ && tile_ok ? (wave ? 4 : 0) : m2l_matrix_ ? 1 : 2;
 }
 
 int Engine::tune(int nrhs, int mode)
