@@ -836,42 +836,55 @@ __global__ __launch_bounds__(64) void k_p2p_s(const int* __restrict__ tbeg, cons
 typedef double v4d __attribute__((ext_vector_type(4)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 
-// The two waves of a matrix-core near-field block: 64 targets each, or, where
-// the chunk holds at most 64, the same targets in both, every second group of
-// 4 sources each, the second wave's sums added through LDS at the end (its
-// SIMD would idle, and the block's serial chain be twice as long).  FP64 only:
-// the FP32 kernels sum a whole tile in one FP32 chain.
+// The waves of a matrix-core near-field block.  FP64: 4 waves, two for each 64
+// targets of the chunk, or, where it holds at most 64, all four for the same
+// targets; those of the same targets take every second (fourth) group of 4
+// sources of a tile and their sums are added through LDS in wave order at the
+// end.  (One wave for 64 targets left the SIMD of the other idle in chunks of
+// few targets and made the block's serial chain longer.)  FP32: 2 waves of 64
+// targets each, a tile being summed in one FP32 chain.
+template <int NW>
 struct WaveSplit {
-  bool share;      // block-uniform
+  int nshare;      // waves of the same targets (block-uniform)
+  int part;        // this wave's number among them
   int base, ng;    // the wave's first target and its 16-target blocks
   int g0, gs;      // its source groups of a tile
-  __device__ WaveSplit(int w, int tn, bool can_share = true)
+  __device__ WaveSplit(int w, int tn)
   {
-    share = can_share && tn <= 64;
-    base = share ? 0 : 64 * w;
+    nshare = NW == 2 ? 1 : tn <= 64 ? NW : NW / 2;
+    part = w % nshare;
+    base = 64 * (w / nshare);
     ng = base < tn ? min(4, (tn - base + 15) >> 4) : 0;
-    g0 = share ? 4 * w : 0;
-    gs = share ? 8 : 4;
+    g0 = 4 * part;
+    gs = 4 * nshare;
   }
-  // acc of wave 0 += acc of wave 1; red: 1024 doubles of LDS, free after a barrier
+  // acc of part 0 += acc of the others; red: 2048 doubles of LDS, free after a barrier
   template <class V>
   __device__ void sum(V (&acc)[4], double* red, int w, int l) const
   {
-    if (!share) return;
-    __syncthreads();
-    if (w == 1)
+    double* const d = red + (nshare == NW ? 0 : w / nshare) * 1024 + l;
+    for (int o = 1; o < nshare; o++) {
+      __syncthreads();
+      if (part == o)
 #pragma unroll
-      for (int i = 0; i < 4; i++)
+        for (int i = 0; i < 4; i++)
 #pragma unroll
-        for (int v = 0; v < 4; v++) red[(i * 4 + v) * 64 + l] = acc[i][v];
-    __syncthreads();
-    if (w == 0)
+          for (int v = 0; v < 4; v++) d[(i * 4 + v) * 64] = acc[i][v];
+      __syncthreads();
+      if (part == 0)
 #pragma unroll
-      for (int i = 0; i < 4; i++)
+        for (int i = 0; i < 4; i++)
 #pragma unroll
-        for (int v = 0; v < 4; v++) acc[i][v] += red[(i * 4 + v) * 64 + l];
+          for (int v = 0; v < 4; v++) acc[i][v] += d[(i * 4 + v) * 64];
+    }
   }
 };
+// FP64: 4 waves and 128 sources a tile, so that a wave has as many groups
+// between two barriers as with 2 waves and 64, and stages half as much.
+// 4M points / 16 right-hand sides: near field 17.2 -> 16.2 ms (34 -> 36 TFLOP/s);
+// clusters at 21, whose longest chain was the kernel's time: L2T / M2T of the
+// first 16 1.07 -> 0.89 ms.
+constexpr int MF64_BS = 256, MF64_TILE = 128;
 
 // One staged source tile against the wave's first NG 16-target column blocks
 // (NG = the blocks that hold targets, so ragged leaves do not pay for empty
@@ -879,8 +892,8 @@ struct WaveSplit {
 // GUARD: the r < 1e-8 exclusion; an entry whose closest pair of distinct
 // points is farther apart than 1e-7 (flag 0 of the set-up's near-field
 // pass: two different leaves, so no equal points either) goes without it.
-template <int NG, bool GUARD = true>
-__device__ __forceinline__ void p2p_tile64(int cnt4, int kk, int col, const double (*s_pos)[TILE],
+template <int NG, bool GUARD = true, int TW = TILE>
+__device__ __forceinline__ void p2p_tile64(int cnt4, int kk, int col, const double (*s_pos)[TW],
                                            const double (*s_den)[16], const double* tx, const double* ty,
                                            const double* tz, v4d* acc, int g0 = 0, int gs = 4)
 {
@@ -938,20 +951,20 @@ __device__ __forceinline__ void p2p_tile32(int cnt4, int kk, int col, const floa
     for (int v = 0; v < 4; v++) acc[i][v] += (double)part[i][v];
 }
 
-__global__ __launch_bounds__(P2P_BS) void k_p2p_mfma111(int nchunk, const int* __restrict__ tbeg,
+__global__ __launch_bounds__(MF64_BS) void k_p2p_mfma111(int nchunk, const int* __restrict__ tbeg,
                                                         const int* __restrict__ tnum, const int* __restrict__ eptr,
                                                         const int2* __restrict__ ent, const int* __restrict__ echk,
                                                         Points src, Targets trg, int roff, KC kc)
 {
   constexpr int NR = 16;
-  __shared__ double s_pos[3][TILE];
-  __shared__ double s_den[TILE][NR];
+  __shared__ double s_pos[3][MF64_TILE];
+  __shared__ double s_den[MF64_TILE][NR];
   const int c = xcd_item(blockIdx.x, nchunk), t = threadIdx.x, w = t >> 6, l = t & 63;
   if (c >= nchunk) return;
   const int col = l & 15, kk = l >> 4;
   const int r0 = roff + blockIdx.y * NR;
   const int tb = tbeg[c], tn = tnum[c];
-  const WaveSplit ws(w, tn);
+  const WaveSplit<4> ws(w, tn);
   const int ng = ws.ng;  // wave-uniform
   double tx[4], ty[4], tz[4];
 #pragma unroll
@@ -969,18 +982,18 @@ __global__ __launch_bounds__(P2P_BS) void k_p2p_mfma111(int nchunk, const int* _
   for (int e = eptr[c]; e < eptr[c + 1]; e++) {
     const int2 se = ent[e];
     const bool guard = !echk || echk[e] != 0;  // block-uniform
-    for (int b0 = 0; b0 < se.y; b0 += TILE) {
-      const int cnt = min(TILE, se.y - b0), cnt4 = (cnt + 3) & ~3;
+    for (int b0 = 0; b0 < se.y; b0 += MF64_TILE) {
+      const int cnt = min(MF64_TILE, se.y - b0), cnt4 = (cnt + 3) & ~3;
       const int j0 = se.x + b0;
       __syncthreads();
-      for (int i = t; i < cnt4; i += P2P_BS) {
+      for (int i = t; i < cnt4; i += MF64_BS) {
         const bool in = i < cnt;
         s_pos[0][i] = in ? src.x[j0 + i] : 0.0;
         s_pos[1][i] = in ? src.y[j0 + i] : 0.0;
         s_pos[2][i] = in ? src.z[j0 + i] : 0.0;
       }
-      stage_den<1, NR, P2P_BS>(s_den, den, src, j0, cnt, t);
-      for (int i = cnt * NR + t; i < cnt4 * NR; i += P2P_BS) s_den[i / NR][i % NR] = 0.0;
+      stage_den<1, NR, MF64_BS>(s_den, den, src, j0, cnt, t);
+      for (int i = cnt * NR + t; i < cnt4 * NR; i += MF64_BS) s_den[i / NR][i % NR] = 0.0;
       __syncthreads();
       if (!guard) {
         if (ng == 4)
@@ -1002,7 +1015,7 @@ __global__ __launch_bounds__(P2P_BS) void k_p2p_mfma111(int nchunk, const int* _
     }
   }
   ws.sum(acc, &s_den[0][0], w, l);
-  if (ws.share ? w > 0 : ng == 0) return;
+  if (ws.part > 0 || ng == 0) return;
 #pragma unroll
   for (int i = 0; i < 4; i++) {
     const int tt = ws.base + 16 * i + col;
@@ -1037,7 +1050,7 @@ __global__ __launch_bounds__(P2P_BS) void k_p2p_mfma111_f32(int nchunk, const in
   const int col = l & 15, kk = l >> 4;
   const int r0 = roff + blockIdx.y * NR;
   const int tb = tbeg[c], tn = tnum[c];
-  const WaveSplit ws(w, tn, false);
+  const WaveSplit<2> ws(w, tn);
   const int ng = ws.ng;  // wave-uniform
   const double ox = trg.x[tb], oy = trg.y[tb], oz = trg.z[tb];
   float tx[4], ty[4], tz[4];
@@ -1496,7 +1509,7 @@ template <int KT, int NR>
 static void p2p_launch(hipStream_t s, int variant, const Near& c, int nb, Points src, Targets trg, int roff, KC kc)
 {
   if (variant >= 2 && KT == 111 && NR == 16 && src.den_rs == 1)
-    hipLaunchKernelGGL(k_p2p_mfma111, dim3(xcd_grid(c.n), nb), dim3(P2P_BS), 0, s, c.n, c.tbeg, c.tnum, c.eptr, c.ent,
+    hipLaunchKernelGGL(k_p2p_mfma111, dim3(xcd_grid(c.n), nb), dim3(MF64_BS), 0, s, c.n, c.tbeg, c.tnum, c.eptr, c.ent,
                        c.chk, src, trg, roff, kc);
   else if (variant == 1)
     hipLaunchKernelGGL((k_p2p_s<KT, NR>), dim3(2 * c.n, nb), dim3(64), 0, s, c.tbeg, c.tnum, c.eptr, c.ent, src, trg,
@@ -1817,7 +1830,7 @@ constexpr int S2P_TILE32 = 160;
 // centre + radius x unit surface, densities from the node's [rhs][pln] row
 // of the downward (kind 0) or upward (kind 1) equivalent densities.
 template <bool F32>
-__global__ __launch_bounds__(P2P_BS) void k_s2p_mfma111(int nchunk, const int* __restrict__ tbeg,
+__global__ __launch_bounds__(F32 ? P2P_BS : MF64_BS) void k_s2p_mfma111(int nchunk, const int* __restrict__ tbeg,
                                                         const int* __restrict__ tnum, const int* __restrict__ eptr,
                                                         const int* __restrict__ enode, const int* __restrict__ ekind,
                                                         const double4* __restrict__ egeom,
@@ -1829,7 +1842,7 @@ __global__ __launch_bounds__(P2P_BS) void k_s2p_mfma111(int nchunk, const int* _
 {
   typedef typename std::conditional<F32, float, double>::type R;
   // FP32: 160 surface points per staged tile, all of an np 6 surface (152) in one
-  constexpr int NR = 16, TL = F32 ? S2P_TILE32 : TILE;
+  constexpr int NR = 16, TL = F32 ? S2P_TILE32 : MF64_TILE, BS = F32 ? P2P_BS : MF64_BS;
   __shared__ R s_pos[3][TL];
   __shared__ __align__(16) R s_den[TL][NR];
   const int c = xcd_item(blockIdx.x, nchunk), t = threadIdx.x, w = t >> 6, l = t & 63;
@@ -1837,7 +1850,7 @@ __global__ __launch_bounds__(P2P_BS) void k_s2p_mfma111(int nchunk, const int* _
   const int col = l & 15, kk = l >> 4;
   const int r0 = roff + blockIdx.y * NR;
   const int tb = tbeg[c], tn = tnum[c];
-  const WaveSplit ws(w, tn, !F32);
+  const WaveSplit<BS / 64> ws(w, tn);
   const int ng = ws.ng;  // wave-uniform
   // FP32: coordinates relative to the chunk's first target; FP64: absolute
   const double ox = F32 ? trg.x[tb] : 0.0, oy = F32 ? trg.y[tb] : 0.0, oz = F32 ? trg.z[tb] : 0.0;
@@ -1866,14 +1879,14 @@ __global__ __launch_bounds__(P2P_BS) void k_s2p_mfma111(int nchunk, const int* _
     for (int b0 = 0; b0 < nsp; b0 += TL) {
       const int cnt = min(TL, nsp - b0), cnt4 = (cnt + 3) & ~3;
       __syncthreads();
-      for (int i = t; i < cnt4; i += P2P_BS) {
+      for (int i = t; i < cnt4; i += BS) {
         const bool in = i < cnt;
         const int pi = in ? b0 + i : 0;
         s_pos[0][i] = in ? (R)(g.x + g.w * unit[3 * pi] - ox) : (R)0;
         s_pos[1][i] = in ? (R)(g.y + g.w * unit[3 * pi + 1] - oy) : (R)0;
         s_pos[2][i] = in ? (R)(g.z + g.w * unit[3 * pi + 2] - oz) : (R)0;
       }
-      for (int i = t; i < cnt4 * NR; i += P2P_BS) {
+      for (int i = t; i < cnt4 * NR; i += BS) {
         const int q = i / cnt4, jj = i - q * cnt4;
         s_den[jj][q] = jj < cnt && q < nrv ? (R)buf[(long)q * pln + b0 + jj] : (R)0;
       }
@@ -1893,22 +1906,22 @@ __global__ __launch_bounds__(P2P_BS) void k_s2p_mfma111(int nchunk, const int* _
                         (const float*)ty, (const float*)tz, acc64);
       } else {
         if (ng == 4)
-          p2p_tile64<4>(cnt4, kk, col, (const double(*)[TILE])s_pos, (const double(*)[16])s_den, (const double*)tx,
+          p2p_tile64<4, true, TL>(cnt4, kk, col, (const double(*)[TL])s_pos, (const double(*)[16])s_den, (const double*)tx,
                         (const double*)ty, (const double*)tz, accm, ws.g0, ws.gs);
         else if (ng == 3)
-          p2p_tile64<3>(cnt4, kk, col, (const double(*)[TILE])s_pos, (const double(*)[16])s_den, (const double*)tx,
+          p2p_tile64<3, true, TL>(cnt4, kk, col, (const double(*)[TL])s_pos, (const double(*)[16])s_den, (const double*)tx,
                         (const double*)ty, (const double*)tz, accm, ws.g0, ws.gs);
         else if (ng == 2)
-          p2p_tile64<2>(cnt4, kk, col, (const double(*)[TILE])s_pos, (const double(*)[16])s_den, (const double*)tx,
+          p2p_tile64<2, true, TL>(cnt4, kk, col, (const double(*)[TL])s_pos, (const double(*)[16])s_den, (const double*)tx,
                         (const double*)ty, (const double*)tz, accm, ws.g0, ws.gs);
         else if (ng == 1)
-          p2p_tile64<1>(cnt4, kk, col, (const double(*)[TILE])s_pos, (const double(*)[16])s_den, (const double*)tx,
+          p2p_tile64<1, true, TL>(cnt4, kk, col, (const double(*)[TL])s_pos, (const double(*)[16])s_den, (const double*)tx,
                         (const double*)ty, (const double*)tz, accm, ws.g0, ws.gs);
       }
     }
   }
   if constexpr (!F32) ws.sum(accm, &s_den[0][0], w, l);
-  if (ws.share ? w > 0 : ng == 0) return;
+  if (ws.part > 0 || ng == 0) return;
 #pragma unroll
   for (int i = 0; i < 4; i++) {
     const int tt = ws.base + 16 * i + col;
@@ -1944,7 +1957,7 @@ static void s2p_kt(hipStream_t s, const Far& wide, const Far& c, const double* u
     const int roff = r0 + roff0;
     const dim3 grid(c.n, nb), bs(NF_BS);
     if (KT == 111 && NR == 16 && variant == 2)
-      hipLaunchKernelGGL((k_s2p_mfma111<false>), dim3(xcd_grid(c.n), nb), dim3(P2P_BS), 0, s, c.n, c.tbeg, c.tnum,
+      hipLaunchKernelGGL((k_s2p_mfma111<false>), dim3(xcd_grid(c.n), nb), dim3(MF64_BS), 0, s, c.n, c.tbeg, c.tnum,
                          c.eptr, c.node, c.kind, c.geom, unit_de, unit_ue, nsp, dneden, upeden, Rc, pln, trg, roff, kc,
                          16);
     else if (NR == 16)
