@@ -2712,7 +2712,7 @@ static int gemm_split_of(const GemmArgs& a, long nb)
 
 int gemm_split(const GemmArgs& a)
 {
-  if (a.compensated || a.mfma != 2 || a.Kseg % 8 != 0 || a.ngroup <= 0 || a.maxcols <= 0) return 1;
+  if (a.compensated || a.mfma < 2 || a.Kseg % 8 != 0 || a.ngroup <= 0 || a.maxcols <= 0) return 1;
   const long cols = (long)a.maxcols * a.Rc;
   const long nb = a.M <= 64 ? ((cols + 255) / 256) * a.ngroup
                             : ((cols + 64 * GMX_G - 1) / (64 * GMX_G)) * ((a.M + 16 * GMX_RT - 1) / (16 * GMX_RT)) * a.ngroup;
@@ -2730,10 +2730,10 @@ void gemm(hipStream_t s, const GemmArgs& a)
   // wide tiles, with K split over blocks (partials in a.work) when the
   // columns alone give fewer than 2 blocks per CU; 64 x 64 tiles without a
   // workspace
-  if (a.mfma == 2 && a.Kseg % 8 == 0) {
+  if (a.mfma >= 2 && a.Kseg % 8 == 0) {
     int ks = gemm_split(a);
     const long n32 = (long)((a.M + 31) / 32) * ((cols + 31) / 32) * a.ngroup;
-    if (ks > 1 && (a.M > 64 || n32 <= 512)) {
+    if (a.mfma == 2 && ks > 1 && (a.M > 64 || n32 <= 512)) {
       const dim3 grid((unsigned)((cols + 31) / 32), (unsigned)((a.M + 31) / 32), (unsigned)a.ngroup), bs(64 * ks);
       if (ks <= 4)
         hipLaunchKernelGGL(k_gemm_sm<4>, grid, bs, 0, s, a, ks);

@@ -135,7 +135,7 @@ struct GemmArgs {
                     // put, no bscale, not accumulated, M and Kseg multiples of 8; needs sigma), 0: plain FMA
   const double* sigma;  // compensated: start of every row's accumulation, cmp_sigma of its sum of |A|
   int mfma;         // plain form on the FP64 matrix cores (ignored when compensated):
-                    // 2 wide tiles (up to 160 rows x 128 columns), 1 64 x 64 tiles, 0 VALU
+                    // 2 and 3 wide tiles (up to 160 rows x 128 columns), 2 with 32 x 32 ones where K is split, 1 64 x 64 tiles, 0 VALU
   long ctot;        // all columns of the product (ncol x Rc)
   double* work;     // split-K partials, gemm_split(a) x ctot x M doubles (null or too small: no split)
   long work_n;      // capacity of work in doubles

@@ -98,7 +98,7 @@ Engine::Engine(int kt, const double* coefs, int ncoefs, int np, int ptsmax, int 
   if (const char* rb = std::getenv("KIFMM3D_M2L_RB")) m2l_rb_ = std::atoi(rb);
   if (const char* bs = std::getenv("KIFMM3D_M2L_BS")) m2l_bs_ = std::atoi(bs);
   if (const char* v = std::getenv("KIFMM3D_P2P")) p2p_variant_ = std::atoi(v);
-  if (const char* g = std::getenv("KIFMM3D_GEMM")) gemm_mfma_ = std::string(g) == "valu" ? 0 : std::string(g) == "tile64" ? 1 : 2;
+  if (const char* g = std::getenv("KIFMM3D_GEMM")) gemm_mfma_ = std::string(g) == "valu" ? 0 : std::string(g) == "tile64" ? 1 : std::string(g) == "wide" ? 3 : 2;
   if (const char* g = std::getenv("KIFMM3D_GEMM_SPLIT")) split_blocks_ = std::max(1, std::atoi(g));
   if (const char* m = std::getenv("KIFMM3D_M2L")) {
     const std::string v(m);
@@ -861,7 +861,7 @@ void Engine::build_plan()
     P.dc_zero = pool_i(P.I, rows);
   }
   // down pass, top level first (fmm3d_eval.cpp:195-209)
-  const bool fuse_down = pDC == pDE && pDC % 8 == 0 && gemm_mfma_ == 2;
+  const bool fuse_down = pDC == pDE && pDC % 8 == 0 && gemm_mfma_ >= 2;
   for (int L = 2; L < T.nlevel; L++) {
     std::vector<int> all;
     for (int g : by_depth[L])

@@ -1,12 +1,12 @@
-"""Uncompensated products with K split over the waves of a 32 x 32 tile, where
-a level has few columns, against the wide-tile kernel without a split
-(KIFMM3D_GEMM_SPLIT=1): operator rows that leave part of a 32-row tile (56, 152,
-168, 456), 1 to several hundred columns that leave part of a 32-column one,
-absent children, two source buffers and accumulation (mixed form).  The plain
-form's products are kernel matrices: both ways within the parity bar of the
-oracle.  The mixed form applies pseudoinverses without compensation, which the
-order of a sum moves by 1.2e-11 at np 6 (less at np 4): 1e-9 between the two.
+"""Uncompensated products with K split over the waves of a 32 x 32 tile, where a
+level has few columns, against the wide-tile kernel with the same splits
+(KIFMM3D_GEMM=wide): the same operations in the same order, so both forms'
+results agree to the bit, and the plain form's with the oracle at the parity
+bar.  Operator rows that leave part of a 32-row tile (56, 152, 168, 456), 1 to
+several hundred columns that leave part of a 32-column one, absent children,
+two source buffers and accumulation (mixed form).
 """
+import numpy as np
 import pytest
 
 import kifmm3d as K
@@ -23,16 +23,15 @@ def test_split_against_wide(kt, np_, n, nrhs, monkeypatch):
     p, nor = sphere(n, 51) if kt == 321 else (clusters(n, 52), None)
     ctr, rl = ((0.0, 0.0, 0.0), 0) if kt == 321 else ((0.5, 0.5, 0.5), 1)
     out = {}
-    for split in ("", "1"):
-        if split:
-            monkeypatch.setenv("KIFMM3D_GEMM_SPLIT", split)
+    for gemm in ("", "wide"):
+        if gemm:
+            monkeypatch.setenv("KIFMM3D_GEMM", gemm)
         f = make_fmm(kt, np_, 40, 10, ctr, rl, p, nor, p)
         den = densities(n, f.knl.sdof(), nrhs, 53)
         for mode in (K.MODE_PLAIN, K.MODE_MIXED):
-            out[split, mode] = f.eval(den, nrhs=nrhs, mode=mode).reshape(nrhs, -1).copy()
+            out[gemm, mode] = f.eval(den, nrhs=nrhs, mode=mode).reshape(nrhs, -1).copy()
+    for mode in (K.MODE_PLAIN, K.MODE_MIXED):
+        assert np.array_equal(out["", mode], out["wide", mode])
     o = make_oracle(f, kt, np_, 40, 10, ctr, rl, p, nor, p)
     for r in range(nrhs):
-        ref = o.eval(den[r])
-        for split in ("", "1"):
-            assert relerr(out[split, K.MODE_PLAIN][r], ref) <= PARITY
-        assert relerr(out["", K.MODE_MIXED][r], out["1", K.MODE_MIXED][r]) <= 1e-9
+        assert relerr(out["", K.MODE_PLAIN][r], o.eval(den[r])) <= PARITY
