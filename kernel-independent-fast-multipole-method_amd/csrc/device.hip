@@ -12,6 +12,7 @@
 #include <climits>
 #include <cstdlib>
 #include <mutex>
+#include <stdexcept>
 #include <type_traits>
 #include <utility>
 
@@ -833,6 +834,7 @@ __global__ __launch_bounds__(64) void k_p2p_s(const int* __restrict__ tbeg, cons
 // of v_mfma_f64_16x16x4f64: row l/16 + 4v, column l%16).  Source
 // groups are padded to a multiple of 4 with zero densities.  Summation order
 // differs from the scalar kernels only by FP64 rounding.
+typedef double v2d __attribute__((ext_vector_type(2)));
 typedef double v4d __attribute__((ext_vector_type(4)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 
@@ -2068,164 +2070,155 @@ __global__ __launch_bounds__(256) void k_gemm(GemmArgs p)
   }
 }
 
-// Compensated product y = A x for the pseudoinverse applies, in about twice
-// FP64's precision at four vector operations per multiply-add.
+// Compensated product y = A x for the pseudoinverse applies: every output is an
+// unevaluated sum hi + lo, rounded once at the end.
 //
-// A running sum kept in one binade splits off its own rounding errors: with
-// hi in [2^m, 2^(m+1)) every h = fma(a, b, hi) is a multiple of the fixed
-// u = 2^(m-52), so hi - h is exact, and fma(a, b, hi - h) is the part of a b
-// that h did not take, at most u / 2, rounded to 2^-53 of itself.  lo collects
-// these.  The sum starts at sigma = 1.5 2^m and stays in the binade because
-// the columns of B are scaled by a power of two to at most 1 in magnitude (2
-// at the very top of the FP64 range) and 2^(m-2) bounds the row's sum of |A|
-// (cmp_sigma, once per operator at set-up); hi - sigma is exact and
-// (hi - sigma) + lo rounds once.  The error before that rounding is of the
-// order of K^2 2^-106 sigma, as that of a TwoProd / TwoSum dot product, which
-// takes ten operations instead of four.
+// Dot2 (Ogita, Rump and Oishi, SIAM J. Sci. Comput. 26, 2005): p = fl(a b) is
+// added to hi with TwoSum (Knuth), whose error and that of p are added to lo.
+// fma(a, b, -bb), with bb the part of p that the sum took, is the rest of p and
+// its error in one rounding, so a multiply-add takes eight vector operations.
 //
-// Bound by the FP64 vector rate (the matrix cores do not give out the
-// rounding errors of their sums).  A block of WM x WN x WK waves forms a
-// 32 WM x 32 WN tile, each wave 32 x 32 of it as 4 x 4 per lane (4 LDS reads
-// of 16 bytes feed 64 vector operations), the K steps of 8 double-buffered in
-// LDS; WK > 1 splits K over the block's waves, whose (hi - sigma) --
-// multiples of u, summed exactly -- and lo are added through LDS in wave
-// order, so the result does not depend on scheduling and needs no workspace
-// or second launch.
-// Measured against a TwoProd / TwoSum product on 64 x 64 tiles with no split:
-// 152 x 296 over 524,288 columns (Laplace np 6, 4M points, 16 right-hand
-// sides) 9.36 -> 3.79 ms + 0.26 ms for the scales (27 of 39 T vector
-// operations/s); 608 x 888 (Stokes np 6) over 4,100 columns 970 -> 392 us,
-// over 20 columns 437 -> 55 us; 56 x 152 (np 4) over 64 columns 80 -> 17 us.
-__device__ inline void cmp_acc(double& hi, double& lo, double a, double b)
+// Blocks of 8 products (five and a half operations each).  hi starts at
+// sigma >= 2 S, S = (sum of the block's |a|) (max of its |b|), so it stays in
+// [S, 3 S] and every h = fma(a, b, hi) lies in [hi / 2, 2 hi]: hi - h is exact
+// (Sterbenz), and fma(a, b, hi - h) is what h did not take, at most an ulp / 2
+// of 3 S, rounded to 2^-53 of itself.  hi - sigma is exact for the same reason;
+// it and the sum of the rests are added to the running hi + lo.  In units of
+// 2^-106, and with n blocks, the error is at most 160 sum S + (n + 2)^2 R / 2,
+// R the largest partial sum, against K^2 sum |a b| of Dot2.
+// Which one: blocks where that is no less accurate.  On the translation
+// operators and the check values of evaluates, the largest error before the last
+// rounding over 2^-106 sum |a b| is (Dot2 / blocks) 1.6 / 7.9 at K = 56, 2.6 /
+// 4.3 at 152, 3.8 / 3.6 at 168, 2.9 / 1.8 and 3.7 / 2.5 at 296, 7.4 / 3.3 at 456,
+// 12.3 / 3.0 at 888, 12.7 / 2.2 at 1464; the root mean square is at most 1.3 times
+// Dot2's at 296, 1.1 times at 456 and below it above.  Both round all sampled
+// results correctly; one running sum with a single sigma for all of K was off by
+// up to 8e4 there and misrounded 0.3 % of the results at K = 1464.
+__device__ inline void dot2_acc(double& hi, double& lo, double a, double b)
 {
 #pragma clang fp contract(off)
-  const double h = fma(a, b, hi);
-  lo += fma(a, b, hi - h);
+  const double s = hi + a * b, bb = s - hi, y = hi - (s - bb);
+  lo += y + fma(a, b, -bb);
+  hi = s;
+}
+
+// hi + lo += (h - sigma) + w, of a block that started at sigma
+__device__ inline void cmp_add(double& hi, double& lo, double h, double sigma, double w)
+{
+#pragma clang fp contract(off)  // sigma itself, not the product it was rounded from, is subtracted
+  const double v = h - sigma, s = hi + v, bb = s - hi, r = w + ((hi - (s - bb)) + (v - bb));
+  hi = s + r;
+  lo += r - (hi - s);
+}
+
+// the part of a b that the running sum of a block does not take
+__device__ inline double cmp_rest(double& hi, double a, double b)
+{
+#pragma clang fp contract(off)
+  const double h = fma(a, b, hi), r = fma(a, b, hi - h);
   hi = h;
+  return r;
 }
 
-double cmp_sigma(double abs_row_sum)
+// max over the 4 lanes of a quad
+__device__ inline int quad_max(int v)
 {
-  int m = 0;
-  std::frexp(abs_row_sum, &m);  // abs_row_sum <= 2^m
-  return abs_row_sum > 0.0 ? std::ldexp(1.5, m + 2) : 1.0;
+  v = max(v, __builtin_amdgcn_mov_dpp(v, 0xb1, 0xf, 0xf, true));         // lanes 1 0 3 2
+  return max(v, __builtin_amdgcn_mov_dpp(v, 0x4e, 0xf, 0xf, true));      // lanes 2 3 0 1
 }
 
-// e with 2^e >= m, for the largest magnitude m of a column (0 for a column
-// that is all zero or not finite, whose products are then what they are)
-__device__ inline int cmp_exp(double m)
+bool cmp_blocks(int K) { return K >= 256; }
+
+void cmp_bounds(const double* A, int M, int K, double* out)
 {
-  int e = 0;
-  if (m > 0.0 && m <= DBL_MAX) (void)frexp(m, &e);
-  return min(max(e, -1000), 1023);
+  for (long e = 0; e < (long)M * (K / 8); e++) out[e] = 0.0;
+  for (int k = 0; k < K; k++)
+    for (int i = 0; i < M; i++) out[(long)(k / 8) * M + i] += std::fabs(A[(long)k * M + i]);
+  for (long e = 0; e < (long)M * (K / 8); e++) out[e] *= 2.0 + 1e-9;  // over the rounding of the sum and of hi
 }
 
-// cmp_exp of every column of B, one wave per column
-__global__ __launch_bounds__(256) void k_gemm_cmp_exp(GemmArgs p, int* __restrict__ out)
+// Bound by the FP64 vector rate (the matrix cores do not give out the rounding
+// errors of their sums).  A block of WN x WK waves forms a 32 x 32 WN tile, each
+// wave 32 x 32 of it as 4 x 4 per lane, the K steps of 8 (the blocks above)
+// double-buffered in LDS; BLK takes two columns of a lane through a step at a
+// time, so that the running sums of a block fit beside the 16 hi + lo (234 to 248
+// VGPRs, no scratch).  WK > 1 splits K over the block's waves, whose hi + lo are
+// added through LDS in wave order, so the result does not depend on scheduling
+// and needs no workspace or second launch.
+// Measured against Dot2 on 64 x 64 tiles with no split: 152 x 296 over 524,288
+// columns (Laplace np 6, 4M points, 16 right-hand sides) 9.36 -> 5.1 ms, 152 x 152
+// over them 3.2 (27 and 32 of 39 T vector operations/s); 608 x 888 (Stokes np 6)
+// over 4,100 columns 970 -> 470 us, over 20 columns 437 -> 49 us; 56 x 152 (np 4)
+// over 64 columns 80 -> 15 us.
+template <int WN, int WK, bool BLK>
+__global__ __launch_bounds__(64 * WN * WK, BLK ? 2 : 3) void k_gemm_cmp(GemmArgs p)
 {
-  const long j = (long)blockIdx.x * 4 + (threadIdx.x >> 6), l = threadIdx.x & 63;
-  if (j >= (long)p.ncol * p.Rc) return;  // wave-uniform
-  const long n = j / p.Rc;
-  const double* b = p.B + ((long)p.bnode[n] * p.Rc + (j - n * p.Rc)) * p.Kseg;
-  double m = 0.0;
-  for (long k = 2 * l; k < p.Kseg; k += 128) {
-    const double2 v = *(const double2*)(b + k);
-    m = fmax(m, fmax(fabs(v.x), fabs(v.y)));
-  }
-#pragma unroll
-  for (int d = 1; d < 64; d *= 2) m = fmax(m, __shfl_xor(m, d));
-  if (l == 0) out[j] = cmp_exp(m);
-}
-
-// exps: cmp_exp of every column, or null (the block finds those of its own)
-template <int WM, int WN, int WK>
-__global__ __launch_bounds__(64 * WM * WN * WK, WK == 16 ? 4 : 3) void k_gemm_cmp(GemmArgs p,
-                                                                              const int* __restrict__ exps)
-{
-  static_assert(WK == 1 || (WM == 1 && WN == 1), "K is split between waves of one tile");
-  constexpr int NT = 64 * WM * WN * WK, NG = 64 * WM * WN;   // threads of the block, of one K part
-  constexpr int BM = 32 * WM, BN = 32 * WN, LB = BN + 8;     // LB: padded row, conflict-free staging writes
-  constexpr int NA = (BM * 4 + NG - 1) / NG, NB = BN * 4 / NG;  // 16-byte operand pairs per thread and step
-  constexpr int PART = 16 * (BM + LB);                       // LDS doubles of one K part
+  static_assert(WK == 1 || WN == 1, "K is split between waves of one tile");
+  constexpr int NT = 64 * WN * WK, NG = 64 * WN;  // threads of the block, of one K part
+  constexpr int BM = 32, BN = 32 * WN, LB = BN + 4;  // LB: padded row, conflict-free staging writes
+  constexpr int RW = BLK ? 9 : 8;                    // rows of a staged step: its K indices, the bounds of A and B
+  constexpr int NA = (BM / 2 * RW + NG - 1) / NG, NB = BN * 4 / NG;  // 16-byte operand pairs per thread and step
+  constexpr int PART = 2 * RW * (BM + LB);                           // LDS doubles of one K part
   static_assert(WK == 1 || PART >= 32 * 32, "the split sums reuse the staging memory");
   __shared__ __align__(16) double lds[WK * PART];
-  __shared__ int s_exp[BN];
   const long cb = (long)blockIdx.x * BN, ce = (long)p.ncol * p.Rc;
   const int rb = blockIdx.y * BM, K = p.Kseg, nstep = K / 8;
-  const int t = threadIdx.x, kg = t / NG, tg = t - kg * NG, w = tg >> 6, l = t & 63;
+  const int t = threadIdx.x, kg = t / NG, tg = t % NG, w = tg >> 6, l = t & 63;
   // column c of the block in B (past the end: the last one, whose copies are
   // not stored, as are those of row 0 past the end of A)
   auto column = [&](int c) {
     const long j = min(cb + c, ce - 1), n = j / p.Rc;
     return p.B + ((long)p.bnode[n] * p.Rc + (j - n * p.Rc)) * K;
   };
-  if (exps) {
-    if (t < BN) s_exp[t] = exps[min(cb + t, ce - 1)];
-  } else {
-    constexpr int TPC = NT / BN;  // adjacent threads per column
-    const double* b = column(t / TPC);
-    double m = 0.0;
-#pragma unroll 4
-    for (int k = 2 * (t % TPC); k < K; k += 2 * TPC) {
-      const double2 v = *(const double2*)(b + k);
-      m = fmax(m, fmax(fabs(v.x), fabs(v.y)));
-    }
-#pragma unroll
-    for (int d = 1; d < TPC; d *= 2) m = fmax(m, __shfl_xor(m, d));
-    if (t % TPC == 0) s_exp[t / TPC] = cmp_exp(m);
-  }
-  __syncthreads();
   const int st0 = nstep * kg / WK, st1 = nstep * (kg + 1) / WK;  // this part's K steps
   double* const sA = lds + kg * PART;
-  double* const sB = sA + 16 * BM;
-  int ao[NA];
+  double* const sB = sA + 2 * RW * BM;
+  // staging of A: rows 2 (e % 16), 2 (e % 16) + 1 of K index e / 16 for e = tg + NG i,
+  // K index 8 being the step's bounds
+  const int srow = 2 * (tg % 16), skk = tg / 16, arow = rb + srow < p.M ? rb + srow : 0, ao = skk * p.M + arow;
   const double* bp[NB];
-  double bs[NB];
-#pragma unroll
-  for (int i = 0; i < NA; i++) {  // two rows of one K index
-    const int e = tg + NG * i, row = 2 * (e % (BM / 2)), kk = (e / (BM / 2)) & 7;
-    ao[i] = kk * p.M + (rb + row < p.M ? rb + row : 0);
-  }
 #pragma unroll
   for (int i = 0; i < NB; i++) {  // two K indices of one column
-    const int e = tg + NG * i, c = e >> 2;
-    bp[i] = column(c) + 2 * (e & 3);
-    bs[i] = ldexp(1.0, -s_exp[c]);
+    const int e = tg + NG * i;
+    bp[i] = column(e >> 2) + 2 * (e & 3);
   }
-  double2 ra[NA], rbv[NB];
+  v2d ra[NA], rbv[NB];
   auto load = [&](int st) {
-    const double* a = p.A + (long)st * 8 * p.M;
 #pragma unroll
-    for (int i = 0; i < NA; i++) ra[i] = *(const double2*)(a + ao[i]);
+    for (int i = 0; i < NA; i++) {
+      if (skk + NG / 16 * i < 8)
+        ra[i] = *(const v2d*)(p.A + (long)(st * 8 + NG / 16 * i) * p.M + ao);
+      else if (BLK && skk + NG / 16 * i == 8)
+        ra[i] = *(const v2d*)(p.bound + (long)st * p.M + arow);
+    }
 #pragma unroll
-    for (int i = 0; i < NB; i++) rbv[i] = *(const double2*)(bp[i] + st * 8);
+    for (int i = 0; i < NB; i++) rbv[i] = *(const v2d*)(bp[i] + st * 8);
   };
   auto store = [&](int buf) {
 #pragma unroll
     for (int i = 0; i < NA; i++) {
-      const int e = tg + NG * i, row = 2 * (e % (BM / 2)), kk = e / (BM / 2);
-      if (BM * 4 % NG == 0 || kk < 8) *(double2*)(sA + (buf * 8 + kk) * BM + row) = ra[i];
+      const int kk = skk + NG / 16 * i;
+      if (kk < RW) *(v2d*)(sA + (buf * RW + kk) * BM + srow) = ra[i];
     }
 #pragma unroll
     for (int i = 0; i < NB; i++) {
       const int e = tg + NG * i, c = e >> 2, kk = 2 * (e & 3);
-      sB[(buf * 8 + kk) * LB + c] = rbv[i].x * bs[i];
-      sB[(buf * 8 + kk + 1) * LB + c] = rbv[i].y * bs[i];
+      sB[(buf * RW + kk) * LB + c] = rbv[i].x;
+      sB[(buf * RW + kk + 1) * LB + c] = rbv[i].y;
+      if constexpr (BLK) {  // the column's largest magnitude of the step, from above
+        const int m = quad_max(max(__double2hiint(fabs(rbv[i].x)), __double2hiint(fabs(rbv[i].y))));
+        if (kk == 0) sB[(buf * RW + 8) * LB + c] = __hiloint2double(m, -1);
+      }
     }
   };
   // the wave's tile of the block, and the lane's 4 x 4 of it
-  const int wr = 32 * (w % WM), wc = 32 * (w / WM), r0 = wr + 4 * (l & 7), c0 = wc + 4 * (l >> 3);
-  const bool wact = rb + wr < p.M && cb + wc < ce;  // wave-uniform
-  // M is a multiple of 8: a lane's 4 rows are all in or all past the end
-  const double* sig = p.sigma + (rb + r0 < p.M ? rb + r0 : 0);
+  const int wc = 32 * w, r0 = 4 * (l & 7), c0 = wc + 4 * (l >> 3);
+  const bool wact = cb + wc < ce;  // wave-uniform
   double hi[4][4], lo[4][4];
 #pragma unroll
   for (int i = 0; i < 4; i++)
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-      hi[i][j] = sig[i];
-      lo[i][j] = 0.0;
-    }
+    for (int j = 0; j < 4; j++) hi[i][j] = lo[i][j] = 0.0;
   if (st0 < st1) {
     load(st0);
     store(0);
@@ -2237,99 +2230,146 @@ __global__ __launch_bounds__(64 * WM * WN * WK, WK == 16 ? 4 : 3) void k_gemm_cm
     const bool more = st0 + it + 1 < st1;
     if (more) load(st0 + it + 1);
     if (wact && st0 + it < st1) {
-      const double* pa = sA + buf * 8 * BM + r0;
-      const double* pb = sB + buf * 8 * LB + c0;
-#pragma unroll WK == 16 ? 2 : 8
-      for (int kk = 0; kk < 8; kk++) {
+      const double* pa = sA + buf * RW * BM + r0;
+      const double* pb = sB + buf * RW * LB + c0;
+      auto rows = [&](int kk, double (&a)[4]) {
         const double2 a0 = *(const double2*)(pa + kk * BM), a1 = *(const double2*)(pa + kk * BM + 2);
-        const double2 b0 = *(const double2*)(pb + kk * LB), b1 = *(const double2*)(pb + kk * LB + 2);
-        const double a[4] = {a0.x, a0.y, a1.x, a1.y}, b[4] = {b0.x, b0.y, b1.x, b1.y};
+        a[0] = a0.x; a[1] = a0.y; a[2] = a1.x; a[3] = a1.y;
+      };
+      if constexpr (!BLK) {
+#pragma unroll 2
+        for (int kk = 0; kk < 8; kk++) {
+          double a[4];
+          rows(kk, a);
+          const double2 b0 = *(const double2*)(pb + kk * LB), b1 = *(const double2*)(pb + kk * LB + 2);
+          const double b[4] = {b0.x, b0.y, b1.x, b1.y};
 #pragma unroll
-        for (int i = 0; i < 4; i++)
+          for (int i = 0; i < 4; i++)
 #pragma unroll
-          for (int j = 0; j < 4; j++) cmp_acc(hi[i][j], lo[i][j], a[i], b[j]);
+            for (int j = 0; j < 4; j++) dot2_acc(hi[i][j], lo[i][j], a[i], b[j]);
+        }
+      } else {
+#pragma unroll
+        for (int j0 = 0; j0 < 4; j0 += 2) {
+          double sg[4][2], h[4][2], r[4][2], a[4];
+          rows(8, a);
+#pragma unroll
+          for (int j = 0; j < 2; j++) {
+            const double m = pb[8 * LB + j0 + j];
+#pragma unroll
+            for (int i = 0; i < 4; i++) h[i][j] = sg[i][j] = a[i] * m;
+          }
+#pragma unroll
+          for (int kk = 0; kk < 8; kk += 2) {
+            double a1[4];
+            rows(kk, a);
+            rows(kk + 1, a1);
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+              const double b = pb[kk * LB + j0 + j], b1 = pb[(kk + 1) * LB + j0 + j];
+#pragma unroll
+              for (int i = 0; i < 4; i++) {
+                const double q = cmp_rest(h[i][j], a[i], b), q1 = cmp_rest(h[i][j], a1[i], b1);
+                r[i][j] = kk == 0 ? q + q1 : r[i][j] + (q + q1);
+              }
+            }
+          }
+#pragma unroll
+          for (int j = 0; j < 2; j++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) cmp_add(hi[i][j0 + j], lo[i][j0 + j], h[i][j], sg[i][j], r[i][j]);
+        }
       }
     }
     if (more) store(buf ^ 1);
     __syncthreads();
   }
-  auto result = [&](int c, int row, double h, double lw) {  // the scales are powers of two
-    const double v = ldexp(h + lw, s_exp[c]);
-    return p.cscale ? v * p.cscale[row] : v;
-  };
   auto out_col = [&](int c) {
     const long j = cb + c, n = j / p.Rc;
     return p.C + ((long)p.cnode[n] * p.Rc + (j - n * p.Rc)) * p.M;
   };
+  const double* cs = p.cscale ? p.cscale + rb : nullptr;  // powers of two
   if constexpr (WK == 1) {
-    if (!wact || rb + r0 >= p.M) return;
+    if (!wact || rb + r0 >= p.M) return;  // M is a multiple of 8: a lane's 4 rows are all in or all past the end
 #pragma unroll
     for (int j = 0; j < 4; j++) {
       if (cb + c0 + j >= ce) continue;
       double* out = out_col(c0 + j) + rb + r0;
       double v[4];
 #pragma unroll
-      for (int i = 0; i < 4; i++) v[i] = result(c0 + j, rb + r0 + i, hi[i][j] - sig[i], lo[i][j]);
+      for (int i = 0; i < 4; i++) v[i] = (hi[i][j] + lo[i][j]) * (cs ? cs[r0 + i] : 1.0);
       *(double2*)out = make_double2(v[0], v[1]);
       *(double2*)(out + 2) = make_double2(v[2], v[3]);
     }
   } else {
     constexpr int NE = (32 * 32 + NT - 1) / NT;
-    double h[NE];
-    auto spread = [&](auto&& f) {
-      double* d = lds + kg * 1024;
+    double h[NE], lw[NE];
+    double* const d = lds + kg * 1024 + c0 * 32 + r0;
 #pragma unroll
-      for (int j = 0; j < 4; j++) {
-        *(double2*)(d + (c0 + j) * 32 + r0) = make_double2(f(0, j), f(1, j));
-        *(double2*)(d + (c0 + j) * 32 + r0 + 2) = make_double2(f(2, j), f(3, j));
-      }
-    };
-    spread([&](int i, int j) { return hi[i][j] - sig[i]; });
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < NE; k++) {
-      h[k] = 0.0;
-#pragma unroll
-      for (int g = 0; g < WK; g++) h[k] += lds[g * 1024 + t + NT * k];
+    for (int j = 0; j < 4; j++) {
+      *(double2*)(d + j * 32) = make_double2(hi[0][j], hi[1][j]);
+      *(double2*)(d + j * 32 + 2) = make_double2(hi[2][j], hi[3][j]);
     }
     __syncthreads();
-    spread([&](int i, int j) { return lo[i][j]; });
+#pragma unroll
+    for (int k = 0; k < NE; k++) {
+      h[k] = lds[t + NT * k];
+      lw[k] = 0.0;
+#pragma unroll
+      for (int g = 1; g < WK; g++) {
+#pragma clang fp contract(off)
+        const double v = lds[g * 1024 + t + NT * k], s = h[k] + v, bb = s - h[k];
+        lw[k] += (h[k] - (s - bb)) + (v - bb);
+        h[k] = s;
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      *(double2*)(d + j * 32) = make_double2(lo[0][j], lo[1][j]);
+      *(double2*)(d + j * 32 + 2) = make_double2(lo[2][j], lo[3][j]);
+    }
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < NE; k++) {
-      const int at = t + NT * k, row = rb + (at & 31), c = at >> 5;
-      double lw = 0.0;
+      const int at = t + NT * k, row = at & 31, c = at >> 5;
 #pragma unroll
-      for (int g = 0; g < WK; g++) lw += lds[g * 1024 + at];
-      if (row < p.M && cb + c < ce) out_col(c)[row] = result(c, row, h[k], lw);
+      for (int g = 0; g < WK; g++) lw[k] += lds[g * 1024 + at];
+      if (rb + row < p.M && cb + c < ce) out_col(c)[rb + row] = (h[k] + lw[k]) * (cs ? cs[row] : 1.0);
     }
   }
 }
 
-// The rule by the number of 32 x 32 tiles: 768 blocks of 4 waves at 3 waves
-// per SIMD fill the chip, so below about that count K is split over 16 (8)
-// waves of one block to have enough waves at all; from there on 4 waves per
-// tile keep the blocks small and even (4,100 columns of 608 x 888: 437 us
-// against the 970 of whole 64 x 64 tiles), until 8,192 tiles, where a 32 x 128
-// tile reads each operand of B less often (4M points: 3.79 ms, 64 x 64 tiles
-// whose third row block is half empty 4.07 ms).  The scales: in the block
-// itself where there are few tiles (a launch costs as much), in a pass of
-// their own, kept in the split-K workspace, where 5 to 28 row tiles would
-// each read the columns again (608 x 888: 437 -> 376 + 7 us).
-static void gemm_cmp(hipStream_t s, const GemmArgs& a, long cols)
+// The rule by the number of 32 x 32 tiles.  Below 256 there is not a tile for
+// every CU: 8 waves a tile (130 tiles of K = 152 16.5 us, with 4 waves 17.2; 156 of
+// K = 456 32 and 37), more do not fit the registers (16 waves, which spill: 8.4 us
+// against 11.4 for 4 tiles).  From there 4 waves, whose blocks share a CU (323
+// tiles of K = 888 55 us, with 8 waves 59; 570 of K = 456 88 and 98), until a 32 x
+// 128 tile fills the chip as well and reads A a fourth as often (7,160 tiles of K =
+// 296 421 us, as 4 waves of one tile 463; 81,920 5.1 and 5.8 ms; but 4,427 of K =
+// 888 882 and 857 us).
+template <bool BLK>
+static void gemm_cmp_t(hipStream_t s, const GemmArgs& a, long cols)
 {
   const long n32 = (long)((a.M + 31) / 32) * ((cols + 31) / 32);
-  int* exps = n32 >= 640 && a.work && a.work_n * 2 >= cols ? (int*)a.work : nullptr;
-  if (exps) hipLaunchKernelGGL(k_gemm_cmp_exp, dim3((unsigned)((cols + 3) / 4)), dim3(256), 0, s, a, exps);
-  const unsigned rows = (unsigned)((a.M + 31) / 32);
-  if (n32 >= 8192)
-    hipLaunchKernelGGL((k_gemm_cmp<1, 4, 1>), dim3((unsigned)((cols + 127) / 128), rows), dim3(256), 0, s, a, exps);
-  else if (n32 >= 640)
-    hipLaunchKernelGGL((k_gemm_cmp<1, 1, 4>), dim3((unsigned)((cols + 31) / 32), rows), dim3(256), 0, s, a, exps);
+  const unsigned rows = (unsigned)((a.M + 31) / 32), c32 = (unsigned)((cols + 31) / 32);
+  if (n32 >= 6144)
+    hipLaunchKernelGGL((k_gemm_cmp<4, 1, BLK>), dim3((unsigned)((cols + 127) / 128), rows), dim3(256), 0, s, a);
   else if (n32 >= 256)
-    hipLaunchKernelGGL((k_gemm_cmp<1, 1, 8>), dim3((unsigned)((cols + 31) / 32), rows), dim3(512), 0, s, a, exps);
+    hipLaunchKernelGGL((k_gemm_cmp<1, 4, BLK>), dim3(c32, rows), dim3(256), 0, s, a);
   else
-    hipLaunchKernelGGL((k_gemm_cmp<1, 1, 16>), dim3((unsigned)((cols + 31) / 32), rows), dim3(1024), 0, s, a, exps);
+    hipLaunchKernelGGL((k_gemm_cmp<1, 8, BLK>), dim3(c32, rows), dim3(512), 0, s, a);
+}
+
+static void gemm_cmp(hipStream_t s, const GemmArgs& a, long cols)
+{
+  if (a.nseg != 1 || a.ngroup != 1 || a.B2 || a.bscale || a.accumulate || a.M % 8 || a.Kseg % 8 ||
+      (cmp_blocks(a.Kseg) && !a.bound))
+    throw std::logic_error("compensated product: unsupported arguments");
+  if (cmp_blocks(a.Kseg))
+    gemm_cmp_t<true>(s, a, cols);
+  else
+    gemm_cmp_t<false>(s, a, cols);
 }
 
 // Plain (uncompensated) form on the FP64 matrix cores: the same 64 x 64 tile

@@ -131,9 +131,9 @@ struct GemmArgs {
   const double* bscale;
   const double* cscale;
   int accumulate;
-  int compensated;  // 1: compensated accumulation (pseudoinverse applies: one segment, one group, A stays
-                    // put, no bscale, not accumulated, M and Kseg multiples of 8; needs sigma), 0: plain FMA
-  const double* sigma;  // compensated: start of every row's accumulation, cmp_sigma of its sum of |A|
+  int compensated;  // 1: compensated accumulation (pseudoinverse applies: one segment, one group, no
+                    // bscale, not accumulated, M and Kseg multiples of 8), 0: plain FMA
+  const double* bound;  // compensated, where cmp_blocks(Kseg): cmp_bounds of A on the device
   int mfma;         // plain form on the FP64 matrix cores (ignored when compensated):
                     // 2 and 3 wide tiles (up to 160 rows x 128 columns), 2 with 32 x 32 ones where K is split, 1 64 x 64 tiles, 0 VALU
   long ctot;        // all columns of the product (ncol x Rc)
@@ -144,9 +144,11 @@ struct GemmArgs {
   int bscale_seg;   // bscale applies to segments >= bscale_seg
 };
 void gemm(hipStream_t s, const GemmArgs& a);
-// Starting value of the compensated accumulation of a row of A: 1.5 2^m with
-// 2^(m - 2) at least the row's sum of |A|.
-double cmp_sigma(double abs_row_sum);
+// Whether a compensated product over K sums blocks of 8 products, and the bounds
+// it then needs of its operator (column-major M x K, host): out[K/8][M], twice
+// the block's sum of |A| in the row.
+bool cmp_blocks(int K);
+void cmp_bounds(const double* A, int M, int K, double* out);
 // K splits the wide-tile product takes for these sizes (1: none).
 int gemm_split(const GemmArgs& a);
 

@@ -300,15 +300,16 @@ void Engine::upload_static()
   uc2ue_.upload(O.uc2ue);
   ue2uc_.upload(O.ue2uc);
   dc2de_.upload(O.dc2de);
-  // starting values of the compensated pseudoinverse applies, per operator row
-  auto sigma = [](const std::vector<double>& a, int m) {
-    std::vector<double> v(m, 0.0);
-    for (size_t k = 0; k < a.size(); k++) v[k % m] += std::fabs(a[k]);
-    for (double& x : v) x = dev::cmp_sigma(x);
+  auto bounds = [](const std::vector<double>& A, int m, int k) {
+    std::vector<double> v;
+    if (dev::cmp_blocks(k)) {
+      v.resize((size_t)m * (k / 8));
+      dev::cmp_bounds(A.data(), m, k, v.data());
+    }
     return v;
   };
-  uc2ue_sig_.upload(sigma(O.uc2ue, O.pln[SURF_UE]));
-  dc2de_sig_.upload(sigma(O.dc2de, O.pln[SURF_DE]));
+  uc2ue_bnd_.upload(bounds(O.uc2ue, O.pln[SURF_UE], O.pln[SURF_UC]));
+  dc2de_bnd_.upload(bounds(O.dc2de, O.pln[SURF_DE], O.pln[SURF_DC]));
   de2dc_.upload(O.de2dc);
   m2l_.upload(O.m2l);
   {  // frequency-major copies for the matrix-core M2L: [C][343][sdof][tdof] complex
@@ -358,7 +359,7 @@ void Engine::upload_static()
     m2me_.alloc((size_t)8 * pUE * pUE);
     dev::GemmArgs a{};
     a.M = pUE; a.Kseg = pUC; a.nseg = 1; a.Rc = 1; a.ngroup = 1; a.maxcols = a.ncol = 8 * pUE;
-    a.A = uc2ue_.p; a.a_gstride = 0; a.sigma = uc2ue_sig_.p;
+    a.A = uc2ue_.p; a.a_gstride = 0; a.bound = uc2ue_bnd_.p;
     a.B = ue2uc_.p; a.bnode = I_.p + plan_.fuse_idx;
     a.C = m2me_.p; a.cnode = I_.p + plan_.fuse_idx; a.gbeg = I_.p + plan_.fuse_idx_g;
     a.compensated = 1;
@@ -375,7 +376,7 @@ void Engine::upload_static()
                             hipMemcpyDeviceToDevice, stream_));
     dev::GemmArgs a{};
     a.M = pDE; a.Kseg = pDC; a.nseg = 1; a.Rc = 1; a.ngroup = 1; a.maxcols = a.ncol = 8 * pDE;
-    a.A = dc2de_.p; a.sigma = dc2de_sig_.p;
+    a.A = dc2de_.p; a.bound = dc2de_bnd_.p;
     a.B = de2dc_.p; a.bnode = I_.p + plan_.fdn_b;
     a.C = l2de_.p; a.cnode = I_.p + plan_.fdn_c; a.gbeg = I_.p + plan_.fdn_g;
     a.compensated = 1;
@@ -1389,7 +1390,7 @@ void Engine::run_chunk(const double* srcden, double* trgval, int rc, int mode, h
     a.cscale = op.cscale >= 0 ? D + op.cscale : nullptr;
     a.accumulate = op.accumulate;
     a.compensated = mixed ? 0 : op.compensated;
-    a.sigma = op.a_which == 0 ? uc2ue_sig_.p : dc2de_sig_.p;
+    a.bound = op.a_which == 0 ? uc2ue_bnd_.p : dc2de_bnd_.p;
     a.mfma = gemm_mfma_;
     a.ctot = (long)op.ncol * rc;
     a.work = gwork_.p;
