@@ -1234,7 +1234,14 @@ int Engine::m2l_form(bool mixed, size_t level, int rc) const
   const std::vector<int>& tf = m2l_form_[mixed ? 1 : 0];
   if (level < tf.size() && tf[level] >= 0 && ((tf[level] != 0 && tf[level] != 4) || tile_ok))
     return tf[level];
-  return m2l_tile_ && tile_ok ? (m2l_wave_ == 1 ? 4 : 0) : m2l_matrix_ ? 1 : 2;
+  // Left to its default: one wave per tile in FP64, on every level (16
+  // right-hand sides, M2L of a pass, block per tile / wave per tile: one tile of
+  // np 4 0.070 / 0.022 ms, 30k cube 0.20 / 0.08, 300k cube 2.68 / 1.58, 200k
+  // clusters 8.3 / 4.3, 200k sphere 5.8 / 3.4, 300k clusters at np 8 24.1 /
+  // 10.4); one block per tile in the mixed form, where the other's FP32 sums run
+  // in another order.
+  const bool wave = m2l_wave_ < 0 ? !mixed : m2l_wave_ != 0;
+  return m2l_tile_ && tile_ok ? (wave ? 4 : 0) : m2l_matrix_ ? 1 : 2;
 }
 
 int Engine::tune(int nrhs, int mode)
@@ -1344,7 +1351,12 @@ int Engine::settings(int mode, int* out, int n) const
   const int rc = last_rc_ > 0 ? last_rc_ : 16;
   const int cnt = 1 + (int)plan_.vlev.size();
   if (out && n > 0) out[0] = near_variant(mixed);
-  for (int l = 0; out && l + 1 < std::min(n, cnt); l++) out[l + 1] = m2l_form(mixed, (size_t)l, rc);
+  const std::vector<int>& tf = m2l_form_[mixed ? 1 : 0];
+  for (size_t l = 0; out && (long)l + 1 < std::min(n, cnt); l++) {
+    out[l + 1] = m2l_form(mixed, l, rc);
+    // before an evaluate, whose right-hand sides choose, a default is reported as 0 for either tiled form
+    if (last_rc_ == 0 && m2l_wave_ < 0 && out[l + 1] == 4 && !(l < tf.size() && tf[l] >= 0)) out[l + 1] = 0;
+  }
   return cnt;
 }
 
@@ -1490,13 +1502,6 @@ void Engine::run_chunk(const double* srcden, double* trgval, int rc, int mode, h
     const VLevel& vl = P.vlev[li];
     const int form = m2l_form(mixed, li, rc);
     const bool tiled = form == 0 || form == 4;
-    // The tiled form's launch shape in FP64 is one wave per tile, on every
-    // level (16 right-hand sides, M2L of a pass, block per tile / wave per
-    // tile: 30k cube 0.20 / 0.08 ms, 300k cube 2.68 / 1.58, 200k clusters 8.3 /
-    // 4.3, 200k sphere 5.8 / 3.4, 300k clusters at np 8 24.1 / 10.4); the mixed
-    // form's stays one block per tile unless form 4 is set: its FP32 sums run
-    // in another order.
-    const bool wave = form == 4 || (form == 0 && !mixed && m2l_wave_ < 0);
     const int layout = tiled ? dev::SPEC_RHS_INNER : form == 1 ? dev::SPEC_DOF_INNER : dev::SPEC_FREQ_INNER;
     const int single = mixed && (form <= 1 || form == 4) ? 1 : 0;
     cur_lvl = (int)li;
@@ -1505,7 +1510,7 @@ void Engine::run_chunk(const double* srcden, double* trgval, int rc, int mode, h
                    layout, (const double2*)tw_.p);
     });
     timed(KIFMM3D_K_M2L, [&] {
-      if (wave) {
+      if (form == 4) {
         // slot vl.nsrc (C x rc float2 or double2: rc or 2 rc doubles per
         // frequency) is the zero slot that absent halo children read
         const long zs = (long)O.C * rc * (single ? 1 : 2);

@@ -227,7 +227,7 @@ class Engine {
   int gemm_mfma_ = 2;  // uncompensated GEMMs: 2 wide matrix-core tiles, or 32 x 32 with K split over waves, 3 wide tiles only (=wide), 1 64x64 tiles (KIFMM3D_GEMM=tile64), 0 VALU (=valu)
   bool m2l_tile_ = true;   // tiled matrix-core M2L for scalar kernels and 16-RHS chunks (KIFMM3D_M2L=matrix|group|pair disables)
   bool m2l_matrix_ = true; // parent-grouped matrix-core M2L otherwise (KIFMM3D_M2L=group|pair disables)
-  int m2l_wave_ = -1;      // untuned tiled M2L: 1 form 4 (KIFMM3D_M2L=wave), -1 form 0, whose FP64 launch shape is one wave per tile, 0 one block per tile in FP64 too (other values)
+  int m2l_wave_ = -1;      // untuned tiled M2L: 1 wave per tile (KIFMM3D_M2L=wave), 0 block per tile (other values), -1 the first in FP64
   int m2l_depth_ = 4;       // ... halo parents its spectra loads run ahead (KIFMM3D_M2L_DEPTH)
   int m2l_fpart_ = 0;       // tiled M2L: frequency blocks dealt to the XCDs (KIFMM3D_M2L_FPART=1)
   hipStream_t stream_ = nullptr;
