@@ -172,7 +172,10 @@ int kifmm3d_direct_device(kifmm3d* h, const double* d_srcden, int nrhs, const in
  * [10] up-pass GEMM flops of the mixed form (inner nodes by the fused
  * UC2UE x UE2UC product), [11] near-field entries the mixed form's FP32 near
  * field leaves to its FP64 pass (closest pair below 1/128 of the FP32 offsets'
- * span or below 1e-7; set by the device set-up, 0 before it). */
+ * span or below 1e-7; set by the device set-up, 0 before it), and the chunks
+ * of targets that the kernels take: [12] near field (up to 128 targets of a
+ * leaf), [13] its FP64 kernels (fewer in leaves with long lists), [14] L2T +
+ * M2T, [15] its FP64 kernels. */
 int kifmm3d_plan_stats(const kifmm3d* h, double* out, int n);
 
 const char* kifmm3d_last_error(const kifmm3d* h);
