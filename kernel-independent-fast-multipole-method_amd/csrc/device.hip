@@ -989,10 +989,10 @@ __global__ __launch_bounds__(MF64_BS) void k_p2p_mfma111(int nchunk, const int* 
       const int j0 = se.x + b0;
       __syncthreads();
       for (int i = t; i < cnt4; i += MF64_BS) {
-        const bool in = i < cnt;
-        s_pos[0][i] = in ? src.x[j0 + i] : 0.0;
-        s_pos[1][i] = in ? src.y[j0 + i] : 0.0;
-        s_pos[2][i] = in ? src.z[j0 + i] : 0.0;
+        const int j = j0 + (i < cnt ? i : 0);  // padding: the tile's first point, zero density
+        s_pos[0][i] = src.x[j];
+        s_pos[1][i] = src.y[j];
+        s_pos[2][i] = src.z[j];
       }
       stage_den<1, NR, MF64_BS>(s_den, den, src, j0, cnt, t);
       for (int i = cnt * NR + t; i < cnt4 * NR; i += MF64_BS) s_den[i / NR][i % NR] = 0.0;
