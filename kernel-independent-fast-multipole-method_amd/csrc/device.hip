@@ -2620,8 +2620,6 @@ __global__ __launch_bounds__(256) void k_gemm_reduce(GemmArgs p, int ks)
 // best of 10x2, 10x1 and 5x4 on the 4M-point Laplace and 1M-point Navier runs)
 constexpr int GMX_RT = 10, GMX_G = 2;
 
-// Splits of K that bring a wide-tile product to about a.split_blocks blocks
-// (default 1024, 4 per CU; 1 = no split; each split keeps at least 4 steps of 8).
 // The same product for few columns: a block forms 32 x 32 of C with one wave per
 // split of K (ks of them, k_gemm_mx's splits in its order of operations, so the
 // two agree to the bit), each wave's A and B operands straight from global
@@ -2740,6 +2738,8 @@ __global__ __launch_bounds__(64 * KS) void k_gemm_sm(GemmArgs p, int ks)
   }
 }
 
+// Splits of K that bring a wide-tile product to about a.split_blocks blocks
+// (default 1024, 4 per CU; 1 = no split; each split keeps at least 4 steps of 8).
 static int gemm_split_of(const GemmArgs& a, long nb)
 {
   const long target = a.split_blocks > 0 ? a.split_blocks : 1024;
@@ -2750,13 +2750,26 @@ static int gemm_split_of(const GemmArgs& a, long nb)
   return (int)std::max<long>(ks, 1);
 }
 
-int gemm_split(const GemmArgs& a)
+static int gemm_split(const GemmArgs& a)
 {
   if (a.compensated || a.mfma < 2 || a.Kseg % 8 != 0 || a.ngroup <= 0 || a.maxcols <= 0) return 1;
   const long cols = (long)a.maxcols * a.Rc;
   const long nb = a.M <= 64 ? ((cols + 255) / 256) * a.ngroup
                             : ((cols + 64 * GMX_G - 1) / (64 * GMX_G)) * ((a.M + 16 * GMX_RT - 1) / (16 * GMX_RT)) * a.ngroup;
   return gemm_split_of(a, nb);
+}
+
+// whether the ks splits are the waves of 32 x 32 tiles, which need no workspace
+static bool gemm_small(const GemmArgs& a, int ks)
+{
+  const long n32 = (long)((a.M + 31) / 32) * (((long)a.maxcols * a.Rc + 31) / 32) * a.ngroup;
+  return a.mfma == 2 && ks > 1 && (a.M > 64 || n32 <= 512);
+}
+
+long gemm_work(const GemmArgs& a)
+{
+  const int ks = gemm_split(a);
+  return ks > 1 && !gemm_small(a, ks) ? ks * a.ctot * a.M : 0;
 }
 
 void gemm(hipStream_t s, const GemmArgs& a)
@@ -2772,8 +2785,7 @@ void gemm(hipStream_t s, const GemmArgs& a)
   // workspace
   if (a.mfma >= 2 && a.Kseg % 8 == 0) {
     int ks = gemm_split(a);
-    const long n32 = (long)((a.M + 31) / 32) * ((cols + 31) / 32) * a.ngroup;
-    if (a.mfma == 2 && ks > 1 && (a.M > 64 || n32 <= 512)) {
+    if (gemm_small(a, ks)) {
       const dim3 grid((unsigned)((cols + 31) / 32), (unsigned)((a.M + 31) / 32), (unsigned)a.ngroup), bs(64 * ks);
       if (ks <= 4)
         hipLaunchKernelGGL(k_gemm_sm<4>, grid, bs, 0, s, a, ks);

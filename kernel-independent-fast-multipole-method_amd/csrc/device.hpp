@@ -137,7 +137,7 @@ struct GemmArgs {
   int mfma;         // plain form on the FP64 matrix cores (ignored when compensated):
                     // 2 and 3 wide tiles (up to 160 rows x 128 columns), 2 with 32 x 32 ones where K is split, 1 64 x 64 tiles, 0 VALU
   long ctot;        // all columns of the product (ncol x Rc)
-  double* work;     // split-K partials, gemm_split(a) x ctot x M doubles (null or too small: no split)
+  double* work;     // split-K partials of the wide tiles, gemm_work(a) doubles (null or too small: no split)
   long work_n;      // capacity of work in doubles
   int split_blocks; // blocks the split-K aims at (0: 1024); lower when other streams share the GPU
   const double* B2; // segments >= 1 read this buffer instead of B (wide-tile plain form only)
@@ -149,8 +149,8 @@ void gemm(hipStream_t s, const GemmArgs& a);
 // the block's sum of |A| in the row.
 bool cmp_blocks(int K);
 void cmp_bounds(const double* A, int M, int K, double* out);
-// K splits the wide-tile product takes for these sizes (1: none).
-int gemm_split(const GemmArgs& a);
+// Doubles of a.work that the product takes for these sizes.
+long gemm_work(const GemmArgs& a);
 
 // r2c of the scaled upward equivalent densities on the (2np)^3 grid into
 // complex spectra, stored as double2 or, with single, as float2, in the layout

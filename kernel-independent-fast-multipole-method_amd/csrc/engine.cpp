@@ -965,7 +965,7 @@ void Engine::work_counts(int rc, size_t cnt[NWORK]) const
   cnt[6] = (size_t)rc * T.tndecnt * O.pln[SURF_DE];
   cnt[7] = (size_t)2 * rc * (plan_.max_vsrc + 1) * mm_.sdof * O.C;  // + the zero slot of the wave-per-tile M2L
   cnt[8] = (size_t)2 * rc * plan_.max_vtrg * mm_.tdof * O.C;
-  // split-K partials of the matrix-core GEMMs with few columns, for every
+  // split-K partials of the wide-tile GEMMs with few columns, for every
   // chunk size up to rc (the last chunk of an evaluate may be smaller)
   size_t gw = 0;
   for (const std::vector<GemmOp>* ops : {&plan_.up, &plan_.up_mixed, &plan_.down, &plan_.down_mixed})
@@ -976,8 +976,8 @@ void Engine::work_counts(int rc, size_t cnt[NWORK]) const
         a.compensated = 0;
         a.mfma = gemm_mfma_;
         a.split_blocks = split_blocks_;
-        const int ks = dev::gemm_split(a);
-        if (ks > 1) gw = std::max(gw, (size_t)ks * op.ncol * r * op.M);
+        a.ctot = (long)op.ncol * r;
+        gw = std::max(gw, (size_t)dev::gemm_work(a));
       }
   cnt[9] = gw;
   cnt[10] = user_.kt == 111 ? (size_t)rc * T.sextcnt : 0;
