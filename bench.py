@@ -50,30 +50,30 @@ DEFAULT = "laplace-uniform-4m-16rhs"
 # kernel time of the run for the HBM-side rate.
 PROFILED = {
     ("laplace-uniform-4m-16rhs", "mixed", 256): ("profiles/laplace-uniform-4m-16rhs_mixed.md", {
-        "m2l": {"busy": 0.770, "read": 7.428, "written": 4.831},
-        "p2p": {"busy": 0.410, "read": 3.406, "written": 0.577},
-        "fft_fwd": {"busy": None, "read": 0.728, "written": 4.822},
-        "fft_inv": {"busy": None, "read": 4.833, "written": 0.728},
-        "s2m": {"busy": 0.318, "read": 0.372, "written": 1.242},
-        "s2p": {"busy": 0.210, "read": 1.285, "written": 0.575},
-        "gemm_up": {"busy": 0.459, "read": None, "written": None},
-        "gemm_down": {"busy": 0.459, "read": None, "written": None},
+        "m2l": {"busy": 0.761, "read": 7.406, "written": 4.831},
+        "p2p": {"busy": 0.405, "read": 3.394, "written": 0.577},
+        "fft_fwd": {"busy": None, "read": 0.729, "written": 4.831},
+        "fft_inv": {"busy": None, "read": 4.831, "written": 0.728},
+        "s2m": {"busy": 0.320, "read": 0.372, "written": 1.242},
+        "s2p": {"busy": 0.212, "read": 1.289, "written": 0.575},
+        "gemm_up": {"busy": 0.472, "read": None, "written": None},
+        "gemm_down": {"busy": 0.472, "read": None, "written": None},
     }),
     ("laplace-uniform-4m-16rhs", "plain", 256): ("profiles/laplace-uniform-4m-16rhs_plain.md", {
-        "m2l": {"busy": 0.823, "read": 19.448, "written": 10.323},
-        "p2p": {"busy": 0.354, "read": 8.106, "written": 0.558},
-        "fft_fwd": {"busy": None, "read": 0.729, "written": 9.662},
+        "m2l": {"busy": 0.817, "read": 19.469, "written": 10.322},
+        "p2p": {"busy": 0.380, "read": 3.581, "written": 0.565},
+        "fft_fwd": {"busy": None, "read": 0.729, "written": 9.661},
         "fft_inv": {"busy": None, "read": 9.662, "written": 0.728},
-        "s2m": {"busy": 0.318, "read": 0.641, "written": 1.245},
-        "s2p": {"busy": 0.260, "read": 1.303, "written": 0.556},
+        "s2m": {"busy": 0.320, "read": 0.641, "written": 1.245},
+        "s2p": {"busy": 0.256, "read": 1.280, "written": 0.540},
     }),
     ("navier-clusters-1m", "mixed", 150): ("profiles/navier-clusters-1m_mixed.md", {
-        "m2l": {"busy": 0.322, "read": 61.435, "written": 3.235},
-        "p2p": {"busy": None, "read": 1.976, "written": 0.026},
+        "m2l": {"busy": 0.420, "read": 4.151, "written": 2.632},
+        "p2p": {"busy": None, "read": 1.720, "written": 0.026},
         "fft_fwd": {"busy": None, "read": 0.210, "written": 1.599},
-        "fft_inv": {"busy": None, "read": 1.896, "written": 0.573},
-        "gemm_up": {"busy": 0.369, "read": None, "written": None},
-        "gemm_down": {"busy": 0.369, "read": None, "written": None},
+        "fft_inv": {"busy": None, "read": 4.689, "written": 0.608},
+        "gemm_up": {"busy": 0.437, "read": None, "written": None},
+        "gemm_down": {"busy": 0.437, "read": None, "written": None},
     }),
 }
 
