@@ -2146,10 +2146,10 @@ void cmp_bounds(const double* A, int M, int K, double* out)
 // added through LDS in wave order, so the result does not depend on scheduling
 // and needs no workspace or second launch.
 // Measured against Dot2 on 64 x 64 tiles with no split: 152 x 296 over 524,288
-// columns (Laplace np 6, 4M points, 16 right-hand sides) 9.36 -> 5.1 ms, 152 x 152
-// over them 3.2 (27 and 32 of 39 T vector operations/s); 608 x 888 (Stokes np 6)
-// over 4,100 columns 970 -> 470 us, over 20 columns 437 -> 49 us; 56 x 152 (np 4)
-// over 64 columns 80 -> 15 us.
+// columns (Laplace np 6, 4M points, 16 right-hand sides) 9.36 -> 5.2 ms, 152 x 152
+// over them 3.2 (vector instructions in 86 and 94 % of the issue slots); 608 x 888
+// (Stokes np 6) over 4,100 columns 970 -> 490 us, over 20 columns 437 -> 49 us; 56
+// x 152 (np 4) over 64 columns 80 -> 15 us.
 template <int WN, int WK, bool BLK>
 __global__ __launch_bounds__(64 * WN * WK, BLK ? 2 : 3) void k_gemm_cmp(GemmArgs p)
 {
@@ -2341,13 +2341,13 @@ __global__ __launch_bounds__(64 * WN * WK, BLK ? 2 : 3) void k_gemm_cmp(GemmArgs
 }
 
 // The rule by the number of 32 x 32 tiles.  Below 256 there is not a tile for
-// every CU: 8 waves a tile (130 tiles of K = 152 16.5 us, with 4 waves 17.2; 156 of
-// K = 456 32 and 37), more do not fit the registers (16 waves, which spill: 8.4 us
-// against 11.4 for 4 tiles).  From there 4 waves, whose blocks share a CU (323
-// tiles of K = 888 55 us, with 8 waves 59; 570 of K = 456 88 and 98), until a 32 x
-// 128 tile fills the chip as well and reads A a fourth as often (7,160 tiles of K =
-// 296 421 us, as 4 waves of one tile 463; 81,920 5.1 and 5.8 ms; but 4,427 of K =
-// 888 882 and 857 us).
+// every CU: 8 waves a tile (200 tiles of K = 152 16.4 us, with 4 waves 17.5; 156 of
+// K = 456 31.5 and 35.6), more do not fit the registers (16 waves, which spill: 4
+// tiles 11.4 us against 8.4).  From there 4 waves, whose blocks share a CU (323
+// tiles of K = 888 53.5 us, with 8 waves 58.8; 570 of K = 456 87.5 and 95.9), until
+// a 32 x 128 tile fills the chip as well and reads A a fourth as often (7,160 tiles
+// of K = 296 440 us, as 4 waves of one tile 498; 81,920 5.2 and 5.8 ms; but 4,427 of
+// K = 888 878 and 845 us).
 template <bool BLK>
 static void gemm_cmp_t(hipStream_t s, const GemmArgs& a, long cols)
 {
