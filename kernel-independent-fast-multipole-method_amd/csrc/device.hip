@@ -15,6 +15,7 @@
 #include <stdexcept>
 #include <type_traits>
 #include <utility>
+#include <vector>
 
 #include "device.hpp"
 
@@ -2083,7 +2084,9 @@ __global__ __launch_bounds__(256) void k_gemm(GemmArgs p)
 // [S, 3 S] and every h = fma(a, b, hi) lies in [hi / 2, 2 hi]: hi - h is exact
 // (Sterbenz), and fma(a, b, hi - h) is what h did not take, at most an ulp / 2
 // of 3 S, rounded to 2^-53 of itself.  hi - sigma is exact for the same reason;
-// it and the sum of the rests are added to the running hi + lo.  In units of
+// it and the sum of the rests are added to the running hi + lo.  B is scaled by a
+// power of two below 1 / (4 row sums of |A|), so that no sum passes the largest
+// |b|: a column of finite values overflows in its result or not at all.  In units of
 // 2^-106, and with n blocks, the error is at most 160 sum S + (n + 2)^2 R / 2,
 // R the largest partial sum, against K^2 sum |a b| of Dot2.
 // Which one: blocks where that is no less accurate.  On the translation
@@ -2129,12 +2132,20 @@ __device__ inline int quad_max(int v)
 
 bool cmp_blocks(int K) { return K >= 256; }
 
-void cmp_bounds(const double* A, int M, int K, double* out)
+double cmp_bounds(const double* A, int M, int K, double* out)
 {
+  std::vector<double> row(M, 0.0);
   for (long e = 0; e < (long)M * (K / 8); e++) out[e] = 0.0;
   for (int k = 0; k < K; k++)
-    for (int i = 0; i < M; i++) out[(long)(k / 8) * M + i] += std::fabs(A[(long)k * M + i]);
+    for (int i = 0; i < M; i++) {
+      const double a = std::fabs(A[(long)k * M + i]);
+      out[(long)(k / 8) * M + i] += a;
+      row[i] += a;
+    }
   for (long e = 0; e < (long)M * (K / 8); e++) out[e] *= 2.0 + 1e-9;  // over the rounding of the sum and of hi
+  int m = 0;
+  std::frexp(4.0 * *std::max_element(row.begin(), row.end()), &m);
+  return std::ldexp(1.0, m);
 }
 
 // Bound by the FP64 vector rate (the matrix cores do not give out the rounding
@@ -2183,6 +2194,7 @@ __global__ __launch_bounds__(64 * WN * WK, BLK ? 2 : 3) void k_gemm_cmp(GemmArgs
     bp[i] = column(e >> 2) + 2 * (e & 3);
   }
   v2d ra[NA], rbv[NB];
+  const double bmul = BLK ? 1.0 / p.bound_scale : 1.0;
   auto load = [&](int st) {
 #pragma unroll
     for (int i = 0; i < NA; i++) {
@@ -2203,6 +2215,7 @@ __global__ __launch_bounds__(64 * WN * WK, BLK ? 2 : 3) void k_gemm_cmp(GemmArgs
 #pragma unroll
     for (int i = 0; i < NB; i++) {
       const int e = tg + NG * i, c = e >> 2, kk = 2 * (e & 3);
+      if constexpr (BLK) rbv[i] *= bmul;
       sB[(buf * RW + kk) * LB + c] = rbv[i].x;
       sB[(buf * RW + kk + 1) * LB + c] = rbv[i].y;
       if constexpr (BLK) {  // the column's largest magnitude of the step, from above
@@ -2288,7 +2301,8 @@ __global__ __launch_bounds__(64 * WN * WK, BLK ? 2 : 3) void k_gemm_cmp(GemmArgs
     const long j = cb + c, n = j / p.Rc;
     return p.C + ((long)p.cnode[n] * p.Rc + (j - n * p.Rc)) * p.M;
   };
-  const double* cs = p.cscale ? p.cscale + rb : nullptr;  // powers of two
+  // powers of two: the level's scale, and back from that of B
+  auto scale = [&](int row) { return (p.cscale ? p.cscale[rb + row] : 1.0) * (BLK ? p.bound_scale : 1.0); };
   if constexpr (WK == 1) {
     if (!wact || rb + r0 >= p.M) return;  // M is a multiple of 8: a lane's 4 rows are all in or all past the end
 #pragma unroll
@@ -2297,7 +2311,7 @@ __global__ __launch_bounds__(64 * WN * WK, BLK ? 2 : 3) void k_gemm_cmp(GemmArgs
       double* out = out_col(c0 + j) + rb + r0;
       double v[4];
 #pragma unroll
-      for (int i = 0; i < 4; i++) v[i] = (hi[i][j] + lo[i][j]) * (cs ? cs[r0 + i] : 1.0);
+      for (int i = 0; i < 4; i++) v[i] = (hi[i][j] + lo[i][j]) * scale(r0 + i);
       *(double2*)out = make_double2(v[0], v[1]);
       *(double2*)(out + 2) = make_double2(v[2], v[3]);
     }
@@ -2335,7 +2349,7 @@ __global__ __launch_bounds__(64 * WN * WK, BLK ? 2 : 3) void k_gemm_cmp(GemmArgs
       const int at = t + NT * k, row = at & 31, c = at >> 5;
 #pragma unroll
       for (int g = 0; g < WK; g++) lw[k] += lds[g * 1024 + at];
-      if (rb + row < p.M && cb + c < ce) out_col(c)[rb + row] = (h[k] + lw[k]) * (cs ? cs[row] : 1.0);
+      if (rb + row < p.M && cb + c < ce) out_col(c)[rb + row] = (h[k] + lw[k]) * scale(row);
     }
   }
 }
@@ -2364,7 +2378,7 @@ static void gemm_cmp_t(hipStream_t s, const GemmArgs& a, long cols)
 static void gemm_cmp(hipStream_t s, const GemmArgs& a, long cols)
 {
   if (a.nseg != 1 || a.ngroup != 1 || a.B2 || a.bscale || a.accumulate || a.M % 8 || a.Kseg % 8 ||
-      (cmp_blocks(a.Kseg) && !a.bound))
+      (cmp_blocks(a.Kseg) && (!a.bound || !(a.bound_scale > 0.0))))
     throw std::logic_error("compensated product: unsupported arguments");
   if (cmp_blocks(a.Kseg))
     gemm_cmp_t<true>(s, a, cols);

@@ -134,6 +134,7 @@ struct GemmArgs {
   int compensated;  // 1: compensated accumulation (pseudoinverse applies: one segment, one group, no
                     // bscale, not accumulated, M and Kseg multiples of 8), 0: plain FMA
   const double* bound;  // compensated, where cmp_blocks(Kseg): cmp_bounds of A on the device
+  double bound_scale;   // and what it returned
   int mfma;         // plain form on the FP64 matrix cores (ignored when compensated):
                     // 2 and 3 wide tiles (up to 160 rows x 128 columns), 2 with 32 x 32 ones where K is split, 1 64 x 64 tiles, 0 VALU
   long ctot;        // all columns of the product (ncol x Rc)
@@ -146,9 +147,10 @@ struct GemmArgs {
 void gemm(hipStream_t s, const GemmArgs& a);
 // Whether a compensated product over K sums blocks of 8 products, and the bounds
 // it then needs of its operator (column-major M x K, host): out[K/8][M], twice
-// the block's sum of |A| in the row.
+// the block's sum of |A| in the row.  Returns a power of two above 4 times the
+// largest row sum of |A|.
 bool cmp_blocks(int K);
-void cmp_bounds(const double* A, int M, int K, double* out);
+double cmp_bounds(const double* A, int M, int K, double* out);
 // Doubles of a.work that the product takes for these sizes.
 long gemm_work(const GemmArgs& a);
 

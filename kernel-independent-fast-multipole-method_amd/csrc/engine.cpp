@@ -300,16 +300,16 @@ void Engine::upload_static()
   uc2ue_.upload(O.uc2ue);
   ue2uc_.upload(O.ue2uc);
   dc2de_.upload(O.dc2de);
-  auto bounds = [](const std::vector<double>& A, int m, int k) {
+  auto bounds = [](const std::vector<double>& A, int m, int k, DVec<double>& dst, double& scale) {
     std::vector<double> v;
     if (dev::cmp_blocks(k)) {
       v.resize((size_t)m * (k / 8));
-      dev::cmp_bounds(A.data(), m, k, v.data());
+      scale = dev::cmp_bounds(A.data(), m, k, v.data());
     }
-    return v;
+    dst.upload(v);
   };
-  uc2ue_bnd_.upload(bounds(O.uc2ue, O.pln[SURF_UE], O.pln[SURF_UC]));
-  dc2de_bnd_.upload(bounds(O.dc2de, O.pln[SURF_DE], O.pln[SURF_DC]));
+  bounds(O.uc2ue, O.pln[SURF_UE], O.pln[SURF_UC], uc2ue_bnd_, bnd_scale_[0]);
+  bounds(O.dc2de, O.pln[SURF_DE], O.pln[SURF_DC], dc2de_bnd_, bnd_scale_[1]);
   de2dc_.upload(O.de2dc);
   m2l_.upload(O.m2l);
   {  // frequency-major copies for the matrix-core M2L: [C][343][sdof][tdof] complex
@@ -359,7 +359,7 @@ void Engine::upload_static()
     m2me_.alloc((size_t)8 * pUE * pUE);
     dev::GemmArgs a{};
     a.M = pUE; a.Kseg = pUC; a.nseg = 1; a.Rc = 1; a.ngroup = 1; a.maxcols = a.ncol = 8 * pUE;
-    a.A = uc2ue_.p; a.a_gstride = 0; a.bound = uc2ue_bnd_.p;
+    a.A = uc2ue_.p; a.a_gstride = 0; a.bound = uc2ue_bnd_.p; a.bound_scale = bnd_scale_[0];
     a.B = ue2uc_.p; a.bnode = I_.p + plan_.fuse_idx;
     a.C = m2me_.p; a.cnode = I_.p + plan_.fuse_idx; a.gbeg = I_.p + plan_.fuse_idx_g;
     a.compensated = 1;
@@ -376,7 +376,7 @@ void Engine::upload_static()
                             hipMemcpyDeviceToDevice, stream_));
     dev::GemmArgs a{};
     a.M = pDE; a.Kseg = pDC; a.nseg = 1; a.Rc = 1; a.ngroup = 1; a.maxcols = a.ncol = 8 * pDE;
-    a.A = dc2de_.p; a.bound = dc2de_bnd_.p;
+    a.A = dc2de_.p; a.bound = dc2de_bnd_.p; a.bound_scale = bnd_scale_[1];
     a.B = de2dc_.p; a.bnode = I_.p + plan_.fdn_b;
     a.C = l2de_.p; a.cnode = I_.p + plan_.fdn_c; a.gbeg = I_.p + plan_.fdn_g;
     a.compensated = 1;
@@ -1405,6 +1405,7 @@ void Engine::run_chunk(const double* srcden, double* trgval, int rc, int mode, h
     a.accumulate = op.accumulate;
     a.compensated = mixed ? 0 : op.compensated;
     a.bound = op.a_which == 0 ? uc2ue_bnd_.p : dc2de_bnd_.p;
+    a.bound_scale = bnd_scale_[op.a_which == 0 ? 0 : 1];
     a.mfma = gemm_mfma_;
     a.ctot = (long)op.ncol * rc;
     a.work = gwork_.p;

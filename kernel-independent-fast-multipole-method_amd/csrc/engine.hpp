@@ -264,6 +264,7 @@ class Engine {
   DVec<double> unit_[4];
   DVec<double> uc2ue_, ue2uc_, dc2de_, de2dc_, m2l_;
   DVec<double> uc2ue_bnd_, dc2de_bnd_;  // dev::cmp_bounds of the operators
+  double bnd_scale_[2] = {1.0, 1.0};
   DVec<double> m2me_;  // 8 blocks of plnUE x plnUE: UC2UE x UE2UC_c (compensated, on the device at setup)
   DVec<double> l2de_;  // 8 blocks of plnDE x 2 plnDC: [DC2DE | DC2DE x DE2DC_c] (plnDC == plnDE)
   DVec<double> opsT_;  // M2L operators as [C][343][sdof][tdof] complex (FP64)
